@@ -20,48 +20,60 @@ void mm_set_error(const char* fmt, ...) {
 extern "C" const char* mm_last_error(void) { return g_err; }
 
 // ---------------------------------------------------------------------------
-// Bulk dequant [K/8, N] -> [K, N] fp16, one thread per packed word.
-// kernels_core.py:747-791 (inline dequant_fp4: grid (N, K/8), 8 rows per
-// thread); bit-exact with src/marlin_gemm.metal:130-185.
+// Bulk dequant [K/8, N] -> [K, N] fp16 (kernels_core.py:747-791; bit-exact with
+// src/marlin_gemm.metal:130-185).  Write-bound: 16 B out per packed word.
+// V adjacent words of one word row per thread.  V = 4 (N % 4 == 0, aligned
+// operands): 16-byte word loads and 8-byte stores, so a wave writes 512
+// contiguous bytes per row: 14336 x 4096 in 26.0 us (5.7 TB/s; a large copy
+// reaches 4.7 TB/s and a fill 6.9).  One word per thread (V = 1, 128 bytes per
+// wave store, the form any other N takes) took 39.5 us.  Without the
+// non-temporal hints 26.6 us.
 // ---------------------------------------------------------------------------
+template <int V, bool INT4>
 __global__ void __launch_bounds__(256)
-k_fp4_dequant(const uint32_t* __restrict__ B, const f16* __restrict__ S,
-              f16* __restrict__ W, int K, int N, int g) {
-  const int n = blockIdx.x * 256 + threadIdx.x;
+k_dequant(const uint32_t* __restrict__ B, const f16* __restrict__ S, const f16* __restrict__ Z,
+          f16* __restrict__ W, int K, int N, int g) {
+  typedef uint32_t wv __attribute__((ext_vector_type(V)));
+  typedef f16 hv __attribute__((ext_vector_type(V)));
+  const int n = (blockIdx.x * 256 + threadIdx.x) * V;
   const int kp = blockIdx.y;
   if (n >= N) return;
-  const uint32_t w = B[(size_t)kp * N + n];
-  const f16 s = S[(size_t)((kp * 8) / g) * N + n];
-  f16* out = W + (size_t)kp * 8 * N + n;
-  if (!__builtin_isfinite((float)s)) {          // reference guard -> +0.0
-#pragma unroll
-    for (int i = 0; i < 8; ++i) out[(size_t)i * N] = (f16)0.0f;
-    return;
-  }
-  const f16x8 v = dq_fp4_word(w, f16x2{s, s});
-#pragma unroll
-  for (int i = 0; i < 8; ++i) out[(size_t)i * N] = v[i];
-}
-
-__global__ void __launch_bounds__(256)
-k_u4_dequant(const uint32_t* __restrict__ B, const f16* __restrict__ S,
-             const f16* __restrict__ Z, f16* __restrict__ W, int K, int N, int g) {
-  const int n = blockIdx.x * 256 + threadIdx.x;
-  const int kp = blockIdx.y;
-  if (n >= N) return;
-  const uint32_t w = B[(size_t)kp * N + n];
   const size_t gi = (size_t)((kp * 8) / g) * N + n;
-  const f16 s = S[gi];
-  const f16 nz = -clamp_zero(Z[gi]);
-  f16* out = W + (size_t)kp * 8 * N + n;
-  if (!__builtin_isfinite((float)s)) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) out[(size_t)i * N] = (f16)0.0f;
-    return;
+  wv w;
+  hv s, z;
+  if constexpr (V == 1) {
+    w[0] = B[(size_t)kp * N + n];
+    s[0] = S[gi];
+    if constexpr (INT4) z[0] = Z[gi];
+  } else {
+    w = __builtin_nontemporal_load((const wv*)(B + (size_t)kp * N + n));
+    s = *(const hv*)(S + gi);
+    if constexpr (INT4) z = *(const hv*)(Z + gi);
   }
-  const f16x8 v = dq_u4_word(w, f16x2{nz, nz}, f16x2{s, s});
+  f16x8 v[V];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) out[(size_t)i * N] = v[i];
+  for (int j = 0; j < V; ++j) {
+    const f16 sj = s[j];
+    if constexpr (INT4) {
+      const f16 nz = -clamp_zero(z[j]);
+      v[j] = dq_u4_word(w[j], f16x2{nz, nz}, f16x2{sj, sj});
+    } else {
+      v[j] = dq_fp4_word(w[j], f16x2{sj, sj});
+    }
+    // reference guard: a non-finite scale gives +0.0
+    if (!__builtin_isfinite((float)sj)) v[j] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  }
+  f16* out = W + (size_t)kp * 8 * N + n;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    hv o;
+#pragma unroll
+    for (int j = 0; j < V; ++j) o[j] = v[j][i];
+    if constexpr (V == 1)
+      out[(size_t)i * N] = o[0];
+    else
+      __builtin_nontemporal_store(o, (hv*)(out + (size_t)i * N));
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -262,6 +274,159 @@ k_u4_quantize(const f16* __restrict__ Wt, int N, int K, int g,
 }
 
 // ---------------------------------------------------------------------------
+// Tiled quantizers (FP4 absmax and asymmetric INT4), same results as
+// k_fp4_quantize / k_u4_quantize.  Those walk a group per thread: adjacent
+// lanes sit K elements apart, so every 2-byte load is a line of its own and the
+// kernel ran at 0.08 TB/s (14336 x 4096 fp16, g = 128: 1700 us).  Here a lane
+// holds the 8 elements of one output word, a wave 512 consecutive k of one row
+// (1 KiB of fp16, read once, kept in registers for both passes), a group's
+// extremes come from the g/8 adjacent lanes that share it, and a 64 x 64-word
+// tile is transposed through LDS so that the words leave as 256-byte runs of
+// the Marlin layout: 36.6 us (4.0 TB/s; a large copy reaches 4.7).  What bounds
+// it is arithmetic as much as memory: with a division and a search over the
+// eight magnitudes per element the same tiling took 60 us.
+// Takes group sizes 8 * 2^i <= 512 and 16-byte aligned weights.
+// ---------------------------------------------------------------------------
+
+// x / a, correctly rounded, for r = RN(1 / a): one Newton step on the quotient
+// with an exact remainder (Markstein, "Computation of elementary functions on
+// the IBM RISC System/6000 processor", 1990).  Its conditions -- no overflow or
+// underflow on the way -- hold for a in [1e-7, 2^100] (both quantizers floor
+// their divisor at 1e-7) and |x| that is zero or at least 2^-80; for fp16 x the
+// latter always holds.
+MM_DEV float div_by(float x, float a, float r) {
+  const float q = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-q, a, x), r, q);
+}
+MM_DEV bool div_ok(float a) { return a <= 0x1p100f; }
+
+// Moves v one step toward zero and sets its last bit: the hardware's
+// round-to-even FP4 convert then sends a midpoint down, as e2m1_nearest does,
+// and leaves every other |v| <= 6 (and not -0) where it was.  Checked against
+// e2m1_nearest over all such floats.
+MM_DEV float fp4_ties_down(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  return __builtin_bit_cast(float, __builtin_elementwise_sub_sat(u, 1u) | 1u);
+}
+template <int BYTE>
+MM_DEV uint32_t fp4_pair(uint32_t word, float v0, float v1) {
+  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(word, fp4_ties_down(v0), fp4_ties_down(v1), 1.0f,
+                                                  BYTE);
+}
+
+constexpr int QT_N = 64;      // rows of W (columns of the packed matrix) per block
+constexpr int QT_WORDS = 64;  // words (8 k) per row and block: one wave-wide load
+constexpr int QT_WAVES = 4;
+constexpr int QT_ROWS = 4;    // rows a wave loads together
+
+template <typename T, bool INT4>
+__global__ void __launch_bounds__(QT_WAVES * 64)
+k_quantize_tile(const T* __restrict__ Wt, int N, int K, int g, uint32_t* __restrict__ B,
+                f16* __restrict__ S, f16* __restrict__ Z) {
+  __shared__ uint32_t words[QT_WORDS][QT_N + 1];
+  __shared__ f16 sc[QT_WORDS][QT_N + 2], zp[INT4 ? QT_WORDS : 1][QT_N + 2];
+  typedef T tvec __attribute__((ext_vector_type(8)));
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n0 = blockIdx.x * QT_N, w0 = blockIdx.y * QT_WORDS;
+  const int wpg = g >> 3;                        // lanes per group, a power of two
+  const int KP = K >> 3;
+  const bool live = w0 + lane < KP;              // whole groups: K % g == 0
+  const int wl = live ? w0 + lane : KP - 1;
+  for (int r0 = wave * QT_ROWS; r0 < QT_N; r0 += QT_WAVES * QT_ROWS) {
+    tvec x[QT_ROWS];
+#pragma unroll
+    for (int i = 0; i < QT_ROWS; ++i)
+      x[i] = *(const tvec*)(Wt + (size_t)min(n0 + r0 + i, N - 1) * K + (size_t)wl * 8);
+#pragma unroll
+    for (int i = 0; i < QT_ROWS; ++i) {
+      uint32_t word = 0;
+      float sv, zv = 0.0f;
+      if constexpr (!INT4) {
+        // |x| bits as integers: NaN sorts above inf, so a NaN in the group wins
+        // as in np.max.
+        uint32_t m = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          m = max(m, __builtin_bit_cast(uint32_t, (float)x[i][j]) & 0x7FFFFFFFu);
+        for (int d = 1; d < wpg; d <<= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d));
+        const float a = m > 0x7F800000u ? __builtin_nanf("")
+                                        : fmaxf(__builtin_bit_cast(float, m), 1e-7f);
+        sv = a / 6.0f;
+        bool ok = div_ok(a);
+        if constexpr (sizeof(T) == 4) {
+          bool tiny = false;
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            tiny |= fabsf((float)x[i][j]) < 0x1p-80f && (float)x[i][j] != 0.0f;
+          ok = ok && !tiny;
+        }
+        if (ok) {
+          const float r = 1.0f / a;
+          float v[8];     // -0 weights come out as +0 (code 0 either way)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[j] = div_by((float)x[i][j], a, r) * 6.0f;
+          word = fp4_pair<0>(word, v[0], v[1]);
+          word = fp4_pair<1>(word, v[2], v[3]);
+          word = fp4_pair<2>(word, v[4], v[5]);
+          word = fp4_pair<3>(word, v[6], v[7]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) word |= e2m1_nearest((float)x[i][j] / a * 6.0f) << (4 * j);
+        }
+      } else {
+        float mn = (float)x[i][0], mx = mn;
+#pragma unroll
+        for (int j = 1; j < 8; ++j) {
+          mn = fminf(mn, (float)x[i][j]);
+          mx = fmaxf(mx, (float)x[i][j]);
+        }
+        for (int d = 1; d < wpg; d <<= 1) {
+          mn = fminf(mn, __shfl_xor(mn, d));
+          mx = fmaxf(mx, __shfl_xor(mx, d));
+        }
+        sv = fmaxf((mx - mn) / 15.0f, 1e-7f);
+        zv = rintf(-mn / sv);
+        if (div_ok(sv)) {
+          const float r = 1.0f / sv;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float q = rintf(div_by((float)x[i][j], sv, r) + zv);
+            word |= (uint32_t)fminf(fmaxf(q, 0.0f), 15.0f) << (4 * j);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float q = rintf((float)x[i][j] / sv + zv);
+            word |= (uint32_t)fminf(fmaxf(q, 0.0f), 15.0f) << (4 * j);
+          }
+        }
+      }
+      words[lane][r0 + i] = word;
+      if ((lane & (wpg - 1)) == 0) {
+        sc[lane / wpg][r0 + i] = (f16)sv;
+        if constexpr (INT4) zp[lane / wpg][r0 + i] = (f16)zv;
+      }
+    }
+  }
+  __syncthreads();
+  const int n = n0 + lane;
+  if (n >= N) return;
+  for (int w = wave; w < QT_WORDS && w0 + w < KP; w += QT_WAVES)
+    B[(size_t)(w0 + w) * N + n] = words[w][lane];
+  for (int q = wave; q < QT_WORDS / wpg && w0 + q * wpg < KP; q += QT_WAVES) {
+    const size_t at = (size_t)(w0 / wpg + q) * N + n;
+    S[at] = sc[q][lane];
+    if constexpr (INT4) Z[at] = zp[q][lane];
+  }
+}
+
+// Rule of the tiled quantizers (see above); other groups and unaligned views
+// take the one-thread-per-group kernels.
+bool quant_tile_ok(const void* W, int g) {
+  return g <= 8 * QT_WORDS && (g & (g - 1)) == 0 && ((uintptr_t)W & 15) == 0;
+}
+
+// ---------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------
 static int check_dims(const char* who, int K, int N, int g) {
@@ -272,29 +437,48 @@ static int check_dims(const char* who, int K, int N, int g) {
   return 0;
 }
 
+template <bool INT4>
+static int launch_dequant(const char* who, const uint32_t* B, const uint16_t* S,
+                          const uint16_t* Z, uint16_t* W, int K, int N, int g, hipStream_t st) {
+  const bool v4 = N % 4 == 0 && ((uintptr_t)B & 15) == 0 &&
+                  (((uintptr_t)S | (uintptr_t)W | (INT4 ? (uintptr_t)Z : 0)) & 7) == 0;
+  const dim3 grid(mm_cdiv(N, v4 ? 1024 : 256), K / 8);
+  if (v4)
+    hipLaunchKernelGGL((k_dequant<4, INT4>), grid, dim3(256), 0, st, B, (const f16*)S,
+                       (const f16*)Z, (f16*)W, K, N, g);
+  else
+    hipLaunchKernelGGL((k_dequant<1, INT4>), grid, dim3(256), 0, st, B, (const f16*)S,
+                       (const f16*)Z, (f16*)W, K, N, g);
+  MM_CHECK_LAUNCH(who);
+  return 0;
+}
+
 extern "C" int mm_fp4_dequant(const uint32_t* B, const uint16_t* S, uint16_t* W, int K, int N,
                               int g, void* stream) {
   if (int rc = check_dims("mm_fp4_dequant", K, N, g)) return rc;
-  dim3 grid(mm_cdiv(N, 256), K / 8);
-  hipLaunchKernelGGL(k_fp4_dequant, grid, dim3(256), 0, (hipStream_t)stream, B,
-                     (const f16*)S, (f16*)W, K, N, g);
-  MM_CHECK_LAUNCH("mm_fp4_dequant");
-  return 0;
+  return launch_dequant<false>("mm_fp4_dequant", B, S, nullptr, W, K, N, g, (hipStream_t)stream);
 }
 
 extern "C" int mm_u4_dequant(const uint32_t* B, const uint16_t* S, const uint16_t* Z, uint16_t* W,
                              int K, int N, int g, void* stream) {
   if (int rc = check_dims("mm_u4_dequant", K, N, g)) return rc;
-  dim3 grid(mm_cdiv(N, 256), K / 8);
-  hipLaunchKernelGGL(k_u4_dequant, grid, dim3(256), 0, (hipStream_t)stream, B, (const f16*)S,
-                     (const f16*)Z, (f16*)W, K, N, g);
-  MM_CHECK_LAUNCH("mm_u4_dequant");
-  return 0;
+  return launch_dequant<true>("mm_u4_dequant", B, S, Z, W, K, N, g, (hipStream_t)stream);
 }
 
 extern "C" int mm_fp4_quantize(const void* W, int w_is_f32, int N, int K, int g, uint32_t* B,
                                uint16_t* S, void* stream) {
   if (int rc = check_dims("mm_fp4_quantize", K, N, g)) return rc;
+  if (quant_tile_ok(W, g)) {
+    const dim3 tiles(mm_cdiv(N, QT_N), mm_cdiv(K / 8, QT_WORDS));
+    if (w_is_f32)
+      hipLaunchKernelGGL((k_quantize_tile<float, false>), tiles, dim3(QT_WAVES * 64), 0,
+                         (hipStream_t)stream, (const float*)W, N, K, g, B, (f16*)S, nullptr);
+    else
+      hipLaunchKernelGGL((k_quantize_tile<f16, false>), tiles, dim3(QT_WAVES * 64), 0,
+                         (hipStream_t)stream, (const f16*)W, N, K, g, B, (f16*)S, nullptr);
+    MM_CHECK_LAUNCH("mm_fp4_quantize");
+    return 0;
+  }
   dim3 grid(mm_cdiv(N, 256), K / g);
   if (w_is_f32)
     hipLaunchKernelGGL(k_fp4_quantize<float>, grid, dim3(256), 0, (hipStream_t)stream,
@@ -330,6 +514,13 @@ extern "C" int mm_fp4_quantize_calibrated(const void* W, int w_is_f32, int N, in
 extern "C" int mm_u4_quantize(const uint16_t* W, int N, int K, int g, uint32_t* B, uint16_t* S,
                               uint16_t* Z, void* stream) {
   if (int rc = check_dims("mm_u4_quantize", K, N, g)) return rc;
+  if (quant_tile_ok(W, g)) {
+    hipLaunchKernelGGL((k_quantize_tile<f16, true>),
+                       dim3(mm_cdiv(N, QT_N), mm_cdiv(K / 8, QT_WORDS)), dim3(QT_WAVES * 64), 0,
+                       (hipStream_t)stream, (const f16*)W, N, K, g, B, (f16*)S, (f16*)Z);
+    MM_CHECK_LAUNCH("mm_u4_quantize");
+    return 0;
+  }
   dim3 grid(mm_cdiv(N, 256), K / g);
   hipLaunchKernelGGL(k_u4_quantize, grid, dim3(256), 0, (hipStream_t)stream, (const f16*)W, N,
                      K, g, B, (f16*)S, (f16*)Z);

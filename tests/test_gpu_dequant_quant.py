@@ -169,3 +169,65 @@ def test_quantize_fp4_calibrated_nan_group_and_bad_percentile(rng):
     assert np.array_equal(packed, rp)
     assert np.array_equal(np.isnan(scales), np.isnan(rs))
     assert np.all(ofp4.unpack_nibbles(rp)[:128, 3] == 8)
+
+
+def _crafted(rng, n, k, dtype):
+    """Weights with ties, signed zeros, subnormals, NaN / inf, a zero row and a
+    constant row (float32 also extreme exponents)."""
+    w = rng.normal(0, 0.02, (n, k)).astype(dtype)
+    w[0] = 0
+    w[min(1, n - 1)] = 0.25
+    w.flat[5 % w.size::97] = -0.0
+    w.flat[11 % w.size::101] = 6e-8
+    ties = np.array([0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0, 6.0], dtype)
+    w[n // 2, :8] = ties
+    w[n // 2, :8][::2] *= -1
+    if n > 4:
+        w[n - 1, k // 2], w[n - 2, 0], w[n - 2, k - 1] = np.nan, np.inf, -np.inf
+        if dtype == np.float32:
+            w[n - 3, ::3], w[n - 4, ::2], w[n - 4, 1::2] = 3e38, 1e-42, -1e-42
+    return w
+
+
+# 8 * 2^i up to 512 run the tiled quantizer; 24 and 1024 the per-group one.
+@pytest.mark.parametrize("N,K,g", [(1, 8, 8), (63, 512, 16), (65, 520, 8), (64, 1536, 512),
+                                   (130, 1152, 128), (66, 544, 32), (33, 768, 256),
+                                   (70, 576, 64), (40, 72, 24), (9, 2048, 1024)])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+def test_quantizers_edges(rng, N, K, g, dtype):
+    import mmfp4
+    w = _crafted(rng, N, K, dtype)
+    announce(f"quantizers N={N} K={K} g={g} {dtype.__name__}")
+    with np.errstate(all="ignore"):
+        rp, rs = ofp4.quantize_fp4(w, g)
+    for view in (0, 1):       # view 1: rows of a tensor that is not 16-byte aligned
+        t = to_dev(w)
+        if view:
+            t = torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(N, K)
+        packed, s = mmfp4.quantize_fp4(t, group_size=g)
+        assert np.array_equal(to_np(packed).view(np.uint32), rp)
+        assert np.array_equal(to_np(s).view(np.uint16), rs.view(np.uint16))
+    if dtype == np.float16:
+        # the reference's uint32 cast of a NaN code is undefined: finite weights
+        w = np.nan_to_num(w, nan=0.01, posinf=0.03, neginf=-0.02)
+        rp, rs, rz = ofp4.pack_u4_weights(w, g)
+        packed, s, z = mmfp4.pack_u4_weights(to_dev(w), group_size=g)
+        assert np.array_equal(to_np(packed).view(np.uint32), rp)
+        assert np.array_equal(to_np(s).view(np.uint16), rs.view(np.uint16))
+        assert np.array_equal(to_np(z), rz)
+
+
+@pytest.mark.parametrize("N", [1, 4, 255, 1020, 1028])
+def test_dequant_widths(rng, N):
+    """Four columns per thread (N % 4 == 0) and one."""
+    import mmfp4
+    K, g = 64, 32
+    packed = rng.integers(0, 2**32, (K // 8, N), dtype=np.uint64).astype(np.uint32)
+    s = rng.normal(0, 0.01, (K // g, N)).astype(np.float16)
+    s[0, 0], s[1, N - 1] = np.inf, np.nan
+    z = rng.integers(0, 16, (K // g, N)).astype(np.float16)
+    announce(f"dequant N={N}")
+    out = to_np(mmfp4.dequant_fp4(to_dev(packed), to_dev(s), K, N, g))
+    assert np.array_equal(out.view(np.uint16), ofp4.dequant_fp4(packed, s, g).view(np.uint16))
+    out = to_np(mmfp4.dequant_int4(to_dev(packed), to_dev(s), to_dev(z), K, N, g))
+    assert np.array_equal(out.view(np.uint16), ofp4.dequant_u4(packed, s, z, g).view(np.uint16))
