@@ -179,8 +179,8 @@ int mm_fp4_gate_up_rowpacked(const uint16_t* A, const uint32_t* Bg, const uint16
 /* Up to three FP4 products sharing A and K, one output each:
  * C[p] [M, N[p]] = A . dequant(B[p], S[p]), p < nmat <= 3 (B[p] Marlin
  * [K/8, N[p]], S[p] [K/g, N[p]]).  The tables are host arrays of device
- * pointers.  M <= 16 runs one launch over all the matrices' column tiles; larger
- * M runs one launch per matrix.  Replaces metal_marlin/kernels_core.py:4875-4948
+ * pointers.  Decode and mid sizes run one launch over all the matrices' column
+ * tiles; larger M runs one launch per matrix.  Replaces metal_marlin/kernels_core.py:4875-4948
  * (mmfp4_fused_qkv) and the Metal shaders/mmfp4_fused_qkv.metal dispatch.
  * Workspace: the larger of mm_gemm_workspace_bytes(M, sum N[p], K) and each
  * mm_gemm_workspace_bytes(M, N[p], K).  Other requirements as mm_fp4_gemm. */

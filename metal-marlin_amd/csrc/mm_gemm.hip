@@ -7,14 +7,16 @@
 // reference's fp16 value (mm_common.h), products accumulate in fp32 on the
 // matrix cores, and the result is rounded once to fp16.
 //
-// Two kernels:
+// Three kernels:
 //  * skinny (M <= 32, decode): weights stream HBM -> registers -> MFMA with no
 //    LDS staging; the M rows ride in a 16-row MFMA operand (zero padded).  A
 //    block holds NW waves that split its K range; the block reduces the waves
 //    in LDS, and a K split across blocks is reduced by the last-arriving block
 //    (deterministic order, counter left at zero for the next call).
-//  * prefill (M > 32): 32x32x16 MFMA tiles, A double-buffered through LDS,
-//    B loaded as packed words one chunk ahead and dequantised in registers.
+//  * mid (M > 32, until the prefill tiles fill the chip): 64- or 128-row tiles
+//    whose waves split K (mm_mid.h).
+//  * prefill: 32x32x16 MFMA tiles of 256 columns over an LDS ring (mm_prefill.h;
+//    k_prefill for shapes outside its 8-column and 64-k pieces).
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -22,6 +24,7 @@
 #include "mm_common.h"
 #include "mm_skinny.h"
 #include "mm_prefill.h"
+#include "mm_mid.h"
 
 // ===========================================================================
 // Skinny path
@@ -644,6 +647,114 @@ k_prefill2(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
   }
 }
 
+// ===========================================================================
+// Mid-sized path (main loop in mm_mid.h): M > 32 up to the sizes where the
+// 256-column prefill tiles fill the chip.  grid = (column tiles, row tiles, K
+// splits).  A K split hands its sums over as k_skinny's does (sc1 partials,
+// an arrival counter per tile, the last block adds the splits in split order):
+// a separate reduction launch costs about 5 us, a quarter of these calls.
+// ===========================================================================
+template <bool INT4, int RB, int WN, bool G128, int ACT>
+__global__ void __launch_bounds__(WN * 256, RB <= 2 ? 4 : 2)
+k_mid(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
+      const f16* __restrict__ S, const f16* __restrict__ Z, const uint32_t* __restrict__ B2,
+      const f16* __restrict__ S2, const f16* __restrict__ Z2, f16* __restrict__ C, int ldc, int M,
+      int N, int K, int g, int cps, float* __restrict__ part, uint32_t* __restrict__ counters,
+      SkMulti mp) {
+  using Sh = mmmid::MidShape<INT4, RB, WN>;
+  constexpr bool PAIR = ACT == SK_SWIGLU || ACT == SK_PAIR;
+  __shared__ __attribute__((aligned(16))) char smem[Sh::LDS_BYTES];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wn = wave % WN, wk = wave / WN;
+  const int l32 = lane & 31, h = lane >> 5;
+  int bx = blockIdx.x;
+  if constexpr (ACT == SK_MULTI) {
+    const int p = bx >= mp.tile0[2] ? 2 : (bx >= mp.tile0[1] ? 1 : 0);
+    B = mp.B[p];
+    S = mp.S[p];
+    Z = mp.Z[p];
+    C = mp.C[p];
+    N = ldc = mp.N[p];
+    bx -= mp.tile0[p];
+  }
+  const int m0 = blockIdx.y * Sh::BM, n0 = bx * (PAIR ? Sh::BN / 2 : Sh::BN);
+  const int c_beg = blockIdx.z * cps, c_end = min(K / mmmid::MID_BK, c_beg + cps);
+  f32x16 acc[RB][2];
+  if constexpr (PAIR) {
+    const PairSrc src{A, lda, M, m0, N, n0, B, B2, S, S2, Z, Z2, N};
+    mmmid::mid_mainloop<INT4, RB, WN, G128, true>(src, K, g, c_beg, c_end, smem, acc);
+  } else {
+    const DenseSrc src{A, lda, M, m0, N, n0, B, S, Z, N};
+    mmmid::mid_mainloop<INT4, RB, WN, G128, false>(src, K, g, c_beg, c_end, smem, acc);
+  }
+  // Wave wk now owns, of every row block, the four rows 8*wk + 4*h + i.
+  f32x4 own[RB][2];
+  mmmid::mid_reduce<RB, WN>(smem, acc, own);
+  const int ks = gridDim.z;
+  if (ks > 1) {
+    const int tile = blockIdx.y * gridDim.x + blockIdx.x;
+    const __amdgpu_buffer_rsrc_t prs =
+        mm_rsrc(part + (size_t)tile * ks * (Sh::BM * Sh::BN));   // this tile's partials
+    auto at = [&](int z, int rb, int j) {
+      return 16u * (uint32_t)((((z * RB + rb) * 2 + j) * (WN * 4) + wave) * 64 + lane);
+    };
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) store_agent_x4(prs, at(blockIdx.z, rb, j), own[rb][j]);
+    __builtin_amdgcn_s_waitcnt(0);   // this wave's partials have reached the coherence point
+    __syncthreads();
+    uint32_t* const s_last = (uint32_t*)smem;
+    if (threadIdx.x == 0) {
+      const uint32_t prev = __hip_atomic_fetch_add(&counters[tile], 1u, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+      *s_last = prev == (uint32_t)ks - 1u;
+    }
+    __syncthreads();
+    if (!*s_last) return;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) own[rb][j] = f32x4{0, 0, 0, 0};
+    for (int z0 = 0; z0 < ks; z0 += 4) {
+      f32x4 ld[4][RB][2];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) ld[i][rb][j] = load_agent_x4(prs, at(min(z0 + i, ks - 1), rb, j));
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (z0 + i < ks)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) own[rb][j] += ld[i][rb][j];
+    }
+    if (threadIdx.x == 0)
+      __hip_atomic_store(&counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  const int ncol = PAIR ? n0 + wn * 32 + l32 : n0 + wn * 64 + 2 * l32;
+  if (ncol >= N) return;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = m0 + rb * 32 + 8 * wk + 4 * h + i;
+      if (row >= M) continue;
+      const float x = own[rb][0][i], y = own[rb][1][i];
+      if constexpr (!PAIR) {
+        *(f16x2*)(C + (size_t)row * ldc + ncol) = f16x2{(f16)x, (f16)y};
+      } else if constexpr (ACT == SK_SWIGLU) {
+        C[(size_t)row * ldc + ncol] = (f16)swiglu(x, y);
+      } else {
+        C[(size_t)row * ldc + ncol] = (f16)x;
+        C[(size_t)row * ldc + N + ncol] = (f16)y;
+      }
+    }
+}
+
 // Sum the K-split partials of the prefill kernel in split order -> fp16 C.
 // Partials are [ks][M][PW]; PW = N, or 2N for the pair modes (gate at n, up
 // at N + n).  SK_SWIGLU writes silu(gate) * up to C [M, N]; the others copy
@@ -951,23 +1062,41 @@ int launch_prefill(const f16* A, int lda, const uint32_t* B, const f16* S, const
 #ifndef MM_PF_KS_BLOCKS
 #define MM_PF_KS_BLOCKS 200   // split K while the grid has fewer blocks than this
 #endif
+// Time of a grid of `blocks` 256-column prefill tiles of `rows` (256 or 128)
+// rows, in us at K = 4096 (it scales with K): one tile per CU, so whole rounds
+// of 256 and a last one that is little cheaper when it is not full.  Fitted to
+// FP4 measurements under sustained load (the clock is power limited):
+//   256 x 256: 96 blocks 98, 192 116, 288 210, 448 241, 512 263, 896 470, 3584 1710
+//   128 x 256: 128 blocks 61, 192 66, 256 73, 264 120, 384 135, 512 152, 1792 508
+double prefill_us(long blocks, int rows) {
+  const long full = blocks / 256, rem = blocks % 256;
+  if (rows == 256) return 3 + 117.0 * full + (rem ? 88 + 0.115 * rem : 0);
+  return 3 + 70.0 * full + (rem ? 54 + 0.07 * rem : 0);
+}
+
 // Prefill plan: tile config (0: 256x256, 1: 128x256, 2: 64x256) and K split.
 struct PrefillPlan {
   int cfg;
   int ksplit;
+  double us;   // at K = 4096, unsplit
 };
 
 PrefillPlan plan_prefill(int M, int N, int K) {
   PrefillPlan p;
   static const int BMs[3] = {256, 128, 64};
-  const long t256 = (long)mm_cdiv(M, 256) * mm_cdiv(N, 256);
-  p.cfg = (M > 128 && t256 >= 240) ? 0 : (M > 64 ? 1 : 2);
-  const long blocks = (long)mm_cdiv(M, BMs[p.cfg]) * mm_cdiv(N, 256);
+  const long ct = mm_cdiv(N, 256);
+  const double big = prefill_us(mm_cdiv(M, 256) * ct, 256);
+  p.us = prefill_us(mm_cdiv(M, 128) * ct, 128);
+  p.cfg = M > 64 ? 1 : 2;
+  if (M > 128 && big < p.us) p.cfg = 0, p.us = big;
+  const long blocks = (long)mm_cdiv(M, BMs[p.cfg]) * ct;
   // Split K when the grid cannot fill the 256 CUs; every split keeps >= 8
-  // chunks of 64 k so the pipeline stays full.
+  // chunks of 64 k so the pipeline stays full.  (256 x 256 tiles are taken only
+  // where one round of them beats two of 128 x 256.)
   const int nch = K / PF2_BK;
   int ks = 1;
-  while (blocks * ks < MM_PF_KS_BLOCKS && nch / (ks * 2) >= 8) ks *= 2;
+  if (p.cfg != 0)
+    while (blocks * ks < MM_PF_KS_BLOCKS && nch / (ks * 2) >= 8) ks *= 2;
   p.ksplit = ks;
   return p;
 }
@@ -975,6 +1104,118 @@ PrefillPlan plan_prefill(int M, int N, int K) {
 size_t prefill_ws_bytes(int M, int N, int K) {
   const PrefillPlan p = plan_prefill(M, N, K);
   return p.ksplit > 1 ? (size_t)p.ksplit * M * N * sizeof(float) : 0;
+}
+
+// Mid plan.  Tiles of 64 rows x 128 columns (8 waves, two blocks per CU), K split
+// while that fits one block per CU and leaves each split 8 chunks; 64 columns
+// where the split grid still leaves half the CUs idle; 128 rows where 65..128
+// rows have more 64-row tiles than CUs.  Measured on MI355X, FP4 g = 128, us
+// before (prefill tiles) -> mid:
+//   M = 64:  4096 -> 2 x 14336 (SwiGLU) 31.5 -> 24.3, 4096 -> 6144 18.8 -> 12.1,
+//            4096 -> 4096 17.0 -> 10.7, 4096 -> 1024 13.9 -> 9.4
+//   M = 100: 4096 -> 2 x 14336 43.1 -> 35.6, 4096 -> 4096 20.9 -> 13.1,
+//            14336 -> 4096 28.0 -> 24.1
+//   M = 512: 4096 -> 4096 31.8 -> 22.1; INT4 4096 -> 6144 59.6 -> 50.5
+// What bounds it is LDS traffic and the matrix cores together.  Its time grows
+// smoothly with the tile count, the prefill tiles' in rounds of 256, so above
+// 128 rows the two are compared (mid_us, prefill_us): M = 512, 4096 -> 6144
+// 48.4 -> 35.7 mid, but M = 2048, 4096 -> 4096 prefill 73 against 81.
+struct MidPlan {
+  int rb, wn;   // 32-row blocks and 64-column groups per tile; wn == 0: not a mid-sized product
+  int ks, cps;  // K splits, chunks per split
+};
+
+// Time of `tiles` 64 x 128 tiles, as prefill_us: 512 tiles 44.6 us, 896 76, 1152 96,
+// 1536 120, 2256 177.
+double mid_us(long tiles) { return 4 + tiles * (20.0 / 256); }
+
+// ct: 128-column tiles of the product (the pair and multi forms count their own).
+MidPlan plan_mid_tiles(int M, long ct, int K) {
+  MidPlan p{2, 0, 1, 0};
+  const int nch = K / mmmid::MID_BK;
+  const long tiles = ct * mm_cdiv(M, 64);
+  if (M <= 32 || K % mmmid::MID_BK != 0 || nch < 4) return p;
+  if (M > 128 && tiles > 256 && mid_us(tiles) > plan_prefill(M, ct * 128, K).us) return p;
+  p.wn = 2;
+  if (M > 64 && M <= 128 && tiles > 256) p.rb = 4;
+  while (tiles * (p.ks + 1) <= 256 && nch / (p.ks + 1) >= 8) ++p.ks;
+  p.cps = mm_cdiv(nch, p.ks);
+  p.ks = mm_cdiv(nch, p.cps);
+  if (tiles * p.ks <= 128) p.wn = 1;
+  return p;
+}
+MidPlan plan_mid(int M, int N, int K) { return plan_mid_tiles(M, mm_cdiv(N, 128), K); }
+
+// Workspace of the plans that a product of these sizes can take: plain over N
+// columns, the pair over 2 x (N / 2), or two or three matrices of N columns in
+// all (up to two more partial tiles).
+size_t mid_ws_bytes(int M, int N, int K) {
+  size_t need = 0;
+  for (long extra = 0; extra <= 2; ++extra) {
+    const long ct = mm_cdiv(N, 128) + extra;
+    const MidPlan p = plan_mid_tiles(M, ct, K);
+    if (p.wn != 0 && p.ks > 1)
+      need = std::max(need, (size_t)p.ks * ct * mm_cdiv(M, 64) * (64 * 128) * sizeof(float));
+  }
+  return need;
+}
+
+template <bool INT4, int ACT, int RB, int WN>
+int launch_mid_tile(const f16* A, const uint32_t* B, const f16* S, const f16* Z,
+                    const uint32_t* B2, const f16* S2, const f16* Z2, f16* C, int ldc, int M,
+                    int N, int K, int g, const MidPlan& p, int gx, void* ws, size_t ws_bytes,
+                    hipStream_t st, const SkMulti* mp) {
+  using Sh = mmmid::MidShape<INT4, RB, WN>;
+  const dim3 grid(gx, mm_cdiv(M, Sh::BM), p.ks);
+  uint32_t* counters = (uint32_t*)ws;
+  float* part = nullptr;
+  if (p.ks > 1) {
+    const size_t need = SK_COUNTER_BYTES + (size_t)p.ks * gx * grid.y * Sh::BM * Sh::BN * 4;
+    MM_CHECK_ARG(ws != nullptr && ws_bytes >= need,
+                 "gemm: workspace of %zu bytes is smaller than the %zu required", ws_bytes, need);
+    part = (float*)((char*)ws + SK_COUNTER_BYTES);
+  }
+  const SkMulti none{};
+  if (g % 128 == 0)
+    hipLaunchKernelGGL((k_mid<INT4, RB, WN, true, ACT>), grid, dim3(Sh::NTHR), 0, st, A, K, B, S,
+                       Z, B2, S2, Z2, C, ldc, M, N, K, g, p.cps, part, counters, mp ? *mp : none);
+  else
+    hipLaunchKernelGGL((k_mid<INT4, RB, WN, false, ACT>), grid, dim3(Sh::NTHR), 0, st, A, K, B, S,
+                       Z, B2, S2, Z2, C, ldc, M, N, K, g, p.cps, part, counters, mp ? *mp : none);
+  MM_CHECK_LAUNCH("gemm(mid)");
+  return 0;
+}
+
+// Whether the operands fit the mid kernel: whole 16-byte pieces of scale rows,
+// one group per 32 k.
+template <bool INT4>
+bool mid_ok(const f16* S, const f16* Z, int N, int g) {
+  return N % 8 == 0 && g % 32 == 0 && (((uintptr_t)S | (INT4 ? (uintptr_t)Z : 0)) & 15) == 0;
+}
+
+// Column tiles per matrix: PLAIN / MULTI 64 * wn columns, pair forms 32 * wn of
+// each.  A K split has at most 256 tiles (plan_mid_tiles), so its counters fit.
+template <bool INT4, int ACT>
+int launch_mid(const MidPlan& p, const f16* A, const uint32_t* B, const f16* S, const f16* Z,
+               const uint32_t* B2, const f16* S2, const f16* Z2, f16* C, int ldc, int M, int N,
+               int K, int g, void* ws, size_t ws_bytes, hipStream_t st, SkMulti* mp = nullptr) {
+  const int bn = 64 * p.wn / (ACT == SK_SWIGLU || ACT == SK_PAIR ? 2 : 1);
+  int gx = mm_cdiv(N, bn);
+  if (ACT == SK_MULTI) {
+    gx = 0;
+    for (int i = 0; i < 3; ++i) {
+      mp->tile0[i] = gx;
+      gx += mm_cdiv(mp->N[i], bn);
+    }
+    mp->tile0[3] = gx;
+  }
+#define MM_LAUNCH_MID(RBV, WNV)                                                                 \
+  return launch_mid_tile<INT4, ACT, RBV, WNV>(A, B, S, Z, B2, S2, Z2, C, ldc, M, N, K, g, p, gx, ws, \
+                                              ws_bytes, st, mp)
+  if (p.rb == 4) MM_LAUNCH_MID(4, 2);
+  if (p.wn == 1) MM_LAUNCH_MID(2, 1);
+  MM_LAUNCH_MID(2, 2);
+#undef MM_LAUNCH_MID
 }
 
 // Row-group height of k_prefill2's tile walk.  One XCD's run of tiles
@@ -1067,6 +1308,9 @@ int gemm_dispatch(const char* who, const f16* A, const uint32_t* B, const f16* S
   if (off32 && M <= 32)
     return launch_skinny<INT4, 2, SK_PLAIN>(A, K, B, Sd, Z, nullptr, nullptr, nullptr, C, N, M, N,
                                             K, g, ws, ws_bytes, st);
+  if (const MidPlan mid = plan_mid(M, N, K); mid.wn != 0 && mid_ok<U4>(S, Z, N, g))
+    return launch_mid<U4, SK_PLAIN>(mid, A, B, S, Z, nullptr, nullptr, nullptr, C, N, M, N, K, g,
+                                    ws, ws_bytes, st);
   // The pipelined kernel stages scale rows in 8-column pieces (N % 8 == 0)
   // and whole 64-k chunks (K % 64 == 0).
   if (N % 8 == 0 && K % PF2_BK == 0) {
@@ -1131,6 +1375,10 @@ int pair_dispatch(const char* who, const f16* A, const uint32_t* Bg, const f16* 
   if (off32 && M <= 32)
     return launch_skinny<INT4, 2, ACT>(A, K, Bg, Sg, Zg, Bu, Su, Zu, C, ldc, M, N, K, g, ws,
                                        ws_bytes, st);
+  if (const MidPlan mid = plan_mid(M, 2 * N, K);
+      mid.wn != 0 && mid_ok<INT4>(Sg, Zg, N, g) && mid_ok<INT4>(Su, Zu, N, g))
+    return launch_mid<INT4, ACT>(mid, A, Bg, Sg, Zg, Bu, Su, Zu, C, ldc, M, N, K, g, ws, ws_bytes,
+                                 st);
   const PrefillPlan p = plan_prefill(M, 2 * N, K);
   float* part = nullptr;
   if (p.ksplit > 1) {
@@ -1154,8 +1402,10 @@ int pair_dispatch(const char* who, const f16* A, const uint32_t* Bg, const f16* 
 }
 
 // Up to three FP4 products sharing A (the Q, K and V projections): decode
-// sizes run one SK_MULTI launch over all their column tiles; larger M runs
-// one launch per matrix.
+// and mid sizes run one SK_MULTI launch over all their column tiles; larger M
+// runs one launch per matrix.  Measured on MI355X, 4096 -> 4096 + 1024 + 1024:
+// M = 32 22.4 us as three launches, 10 as one; M = 100 53 (three launches and
+// their three reductions) -> 18.5.
 int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* const* B,
                    const f16* const* S, f16* const* C, const int* N, int M, int K, int g,
                    void* ws, size_t ws_bytes, hipStream_t st) {
@@ -1183,9 +1433,24 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
   bool off32 = true;
   for (int p = 0; p < nmat; ++p)
     off32 = off32 && (size_t)(K / 8) * (size_t)N[p] * 4 < ((size_t)1 << 32);
-  if (!off32 || M > 16 || flush_steps(g, sk_spw<1>()) == 0 || K % 8 != 0 || g <= 0 ||
-      K % g != 0) {
-    // One product per launch (M > 16, or shapes the GEMM entry rejects with
+  const bool shape_ok = K % 8 == 0 && g > 0 && g % 8 == 0 && K % g == 0;
+  uintptr_t al = (uintptr_t)A;
+  for (int p = 0; p < nmat; ++p) al |= (uintptr_t)B[p] | ((uintptr_t)S[p] & 7) | ((uintptr_t)C[p] & 7);
+  if (M > 32 && shape_ok && (al & 15) == 0) {
+    long ct = 0;
+    bool ok = true;
+    for (int p = 0; p < nmat; ++p) {
+      ct += mm_cdiv(N[p], 128);
+      ok = ok && mid_ok<false>(S[p], nullptr, N[p], g);
+    }
+    const MidPlan mid = plan_mid_tiles(M, ct, K);
+    if (ok && mid.wn != 0)
+      return launch_mid<false, SK_MULTI>(mid, A, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                         nullptr, nullptr, 0, M, ntot, K, g, ws, ws_bytes, st, &mp);
+  }
+  if (!off32 || M > 32 || !shape_ok ||
+      flush_steps(g, M <= 16 ? sk_spw<1>() : sk_spw<2>()) == 0) {
+    // One product per launch (larger M, or shapes the GEMM entry rejects with
     // its own message).
     for (int p = 0; p < nmat; ++p) {
       const int rc = gemm_dispatch<false>(who, A, B[p], S[p], nullptr, C[p], M, N[p], K, g, ws,
@@ -1194,11 +1459,13 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
     }
     return 0;
   }
-  uintptr_t al = (uintptr_t)A;
-  for (int p = 0; p < nmat; ++p) al |= (uintptr_t)B[p] | ((uintptr_t)S[p] & 7) | ((uintptr_t)C[p] & 7);
   MM_CHECK_ARG((al & 15) == 0, "%s: A, B 16-byte / scales, C 8-byte alignment required", who);
   MM_CHECK_ARG(tiles <= SK_MAX_TILES, "%s: too many columns", who);
   if (M == 0) return 0;
+  if (M > 16)
+    return launch_skinny<false, 2, SK_MULTI>(A, K, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                             nullptr, nullptr, 0, M, ntot, K, g, ws, ws_bytes, st,
+                                             &mp);
   return launch_skinny<false, 1, SK_MULTI>(A, K, nullptr, nullptr, nullptr, nullptr, nullptr,
                                            nullptr, nullptr, 0, M, ntot, K, g, ws, ws_bytes, st,
                                            &mp);
@@ -1211,7 +1478,8 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
 // ===========================================================================
 extern "C" size_t mm_gemm_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return SK_COUNTER_BYTES;
-  if (M > 32) return SK_COUNTER_BYTES + prefill_ws_bytes(M, N, K);
+  if (M > 32)
+    return SK_COUNTER_BYTES + std::max(prefill_ws_bytes(M, N, K), mid_ws_bytes(M, N, K));
   // 17..32 rows: enough for the prefill kernel too (the row-packed product
   // takes it from 17 rows).
   if (M > 16) return std::max(skinny_ws_bytes(M, N, K), SK_COUNTER_BYTES + prefill_ws_bytes(M, N, K));

@@ -351,9 +351,10 @@ def mmfp4_fused_qkv(A: torch.Tensor, Q_packed: torch.Tensor, Q_scales: torch.Ten
     """Q, K, V projections sharing A (kernels_core.py:4875-4948):
     Q = A @ dequant(Q_packed, Q_scales), and likewise K and V; packed
     [K/8, N*] Marlin layout, scales [K/group_size, N*].  Returns (Q, K, V)
-    fp16 [M, Nq], [M, Nk], [M, Nv] (shaped like A's leading dims).  M <= 16
-    runs one launch over all three matrices' column tiles; larger M runs one
-    launch per matrix (the reference falls back to separate GEMMs for M > 1)."""
+    fp16 [M, Nq], [M, Nk], [M, Nv] (shaped like A's leading dims).  Decode
+    and mid-sized M run one launch over all three matrices' column tiles;
+    larger M one launch per matrix (the reference falls back to separate GEMMs
+    for M > 1)."""
     dev = _lib.require_device(A, Q_packed, Q_scales, K_packed, K_scales, V_packed, V_scales)
     orig_shape = A.shape
     if A.dim() == 1:

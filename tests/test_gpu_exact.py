@@ -284,3 +284,56 @@ def test_odd_width_bit_exact(rng, M, N):
     q, s, z = _exact_u4(rng, K, N, g)
     _same(mmfp4.marlin_gemm_int4(to_dev(a), to_dev(q), to_dev(s), to_dev(z), g),
           ofp4.gemm_u4_ref(a, q, s, z, g))
+
+
+# The mid-sized kernel (k_mid): rows at and around its 64- and 128-row tiles,
+# columns that end inside a 64-column group or 128-column tile, every scale
+# group per 128-k chunk, K splits with an uneven last split, and the largest
+# row count of 64-column tiles.
+MID = [
+    # (M, K, N, g)
+    (33, 512, 8, 32), (64, 640, 72, 64), (65, 1152, 136, 96), (100, 4096, 1032, 128),
+    (128, 5120, 264, 256), (129, 2176, 1000, 32), (200, 14336, 520, 128),
+    (100, 512, 33024, 128), (500, 1024, 2056, 64), (1000, 2048, 72, 128),
+]
+
+
+@pytest.mark.parametrize("M,K,N,g", MID)
+def test_mid_bit_exact(rng, M, K, N, g):
+    import mmfp4
+    a = _acts(rng, M, K)
+    p, s = _exact_fp4(rng, K, N, g)
+    announce(f"exact mid fp4 M={M} K={K} N={N} g={g}")
+    ref = ofp4.gemm_fp4_ref(a, p, s, g)
+    td = to_dev(a), to_dev(p), to_dev(s)
+    _same(mmfp4.marlin_gemm_fp4(*td, g), ref)
+    # scales 8- but not 16-byte aligned: the prefill kernel's operands
+    sv = torch.cat([td[2].reshape(-1)[:4], td[2].reshape(-1)])[4:].view(td[2].shape)
+    _same(mmfp4.marlin_gemm_fp4(td[0], td[1], sv, g), ref)
+    if N <= 1032:
+        p2, s2 = _exact_fp4(rng, K, N, g)
+        ref2 = ofp4.gemm_fp4_ref(a, p2, s2, g)
+        out = mmfp4.fused_gate_up_gemm(*td, to_dev(p2), to_dev(s2), g)
+        _same(out, np.concatenate([ref, ref2], 1))
+        n3 = max(8, N // 2 // 8 * 8)
+        qkv = mmfp4.mmfp4_fused_qkv(*td, to_dev(p2), to_dev(s2),
+                                    to_dev(p[:, :n3]), to_dev(s[:, :n3]), g)
+        for o, r in zip(qkv, (ref, ref2, ref[:, :n3])):
+            _same(o, r)
+    q, sc, z = _exact_u4(rng, K, N, g)
+    announce(f"exact mid u4 M={M} K={K} N={N} g={g}")
+    _same(mmfp4.marlin_gemm_int4(td[0], to_dev(q), to_dev(sc), to_dev(z), g),
+          ofp4.gemm_u4_ref(a, q, sc, z, g))
+
+
+@pytest.mark.parametrize("M", [17, 24, 32])
+def test_multi_qkv_two_row_blocks(rng, M):
+    """17..32 rows: one launch, bit-identical to one GEMM per matrix."""
+    import mmfp4
+    K, Ns, g = 4096, (4096, 1024, 516), 128
+    w = [_exact_fp4(rng, K, n, g) for n in Ns]
+    a = to_dev(_acts(rng, M, K))
+    args = [to_dev(t) for pair in w for t in pair]
+    announce(f"qkv two row blocks M={M}")
+    for o, (p, s) in zip(mmfp4.mmfp4_fused_qkv(a, *args, g), w):
+        _same(o, ofp4.gemm_fp4_ref(to_np(a), p, s, g))
