@@ -516,7 +516,7 @@ template <int WM, int WN, int RB, bool G64, int STAGES>
 __global__ void __launch_bounds__(WM * WN * 64, MOE_PF_WAVES_PER_SIMD)
 k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
               const int32_t* __restrict__ offsets, int gather, int topk, ExpertW W, int E,
-              int K, int N, int g, int act, int gx, f16* __restrict__ Y) {
+              int K, int N, int g, int act, int gx, int run, f16* __restrict__ Y) {
   constexpr int CW = 2;
   constexpr int SROWS = G64 ? PF2_SROWS_G64 : PF2_SROWS;
   using Sh = Pf2Shape<false, WM, WN, RB, CW, STAGES, SROWS>;
@@ -524,50 +524,64 @@ k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
   // One LDS object only: with a second __shared__ array in the kernel the
   // compiler cannot tell the operand reads from the in-flight global -> LDS
   // copies and waits for all of them (vmcnt(0)) in every chunk, which
-  // serialises the load pipeline.  The row-tile prefix lives past the ring.
-  __shared__ __attribute__((aligned(16))) char smem[Sh::LDS_BYTES + (MOE_MAX_EXPERTS + 1) * 4];
-  int* const tp = (int*)(smem + Sh::LDS_BYTES);   // row-tile prefix over experts
+  // serialises the load pipeline.  The tile prefixes use the ring's memory
+  // before the ring starts.
+  static_assert(Sh::LDS_BYTES >= RB * (MOE_MAX_EXPERTS + 1) * 4 && RB <= WM * WN && WM == 1,
+                "one wave and one prefix per tile class");
+  __shared__ __attribute__((aligned(16))) char smem[Sh::LDS_BYTES];
+  int* const tp = (int*)smem;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / WN, wn = wave % WN;
   const int l32 = lane & 31, h = lane >> 5;
 
-  // tp[e] = row tiles of experts < e (one wave scan).
-  if (wave == 0) {
+  // Row tiles are taken largest first.  Class c holds the tiles with c + 1 live
+  // 32-row blocks: every full tile of an expert is in class RB - 1, its last
+  // partial tile in the class of its rows.  tp[c][e] = class-c tiles of experts
+  // < e (wave c scans class c).  A tile's time is about (2 + live blocks), a
+  // launch has one to two rounds of tiles, and in expert order the CUs that got
+  // a full tile last kept the launch going while the others were idle (CUs busy
+  // 63% of the launch, 82% of a dense one): MM_MOE_LPT.
+  if (wave < RB) {
+    int* const t = tp + wave * (E + 1);
     int base = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + lane;
-      const int t = e < E ? (offsets[e + 1] - offsets[e] + BM - 1) / BM : 0;
-      int incl = t;
+      const int r = e < E ? offsets[e + 1] - offsets[e] : 0;
+      const int part = (r % BM + 31) / 32;
+      const int n = (wave == RB - 1 ? r / BM : 0) + (part == wave + 1 ? 1 : 0);
+      int incl = n;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) {
         const int o = __shfl_up(incl, d);
         if (lane >= d) incl += o;
       }
-      if (e < E) tp[e + 1] = base + incl;
+      if (e < E) t[e + 1] = base + incl;
       base += __shfl(incl, 63);
     }
-    if (lane == 0) tp[0] = 0;
+    if (lane == 0) t[0] = 0;
   }
   __syncthreads();
-  // The grid is an upper bound on gx * (row tiles); blocks past the real
-  // count exit.  Blocks are dealt round-robin to the 8 XCDs, so the linear id
-  // is remapped to give each XCD one contiguous run of (row tile, column
-  // tile) pairs: the column tiles of one row tile then share their A rows in
-  // that XCD's L2.
-  const int nreal = gx * tp[E];
+  // Blocks are dealt round-robin to the 8 XCDs: XCD x takes every eighth run of
+  // `run` row tiles (the tiles an expert has on average, which share its weights
+  // in that XCD's L2), each tile with its gx column tiles, which share its A
+  // rows.  The grid is an upper bound; blocks past the last tile exit.
   const int L = blockIdx.x;
-  if (L >= nreal) return;
-  const int xcd = L & 7, q = nreal >> 3, rem = nreal & 7;
-  const int lin = xcd * q + min(xcd, rem) + (L >> 3);
-  const int y = lin / gx, bx = lin - y * gx;
-  int lo = 0, hi = E - 1;            // expert e with tp[e] <= y < tp[e + 1]
+  const int yx = (L >> 3) / gx, bx = (L >> 3) - yx * gx;
+  int y = (yx / run * 8 + (L & 7)) * run + yx % run;
+  int c = RB - 1;
+  while (c >= 0 && y >= tp[c * (E + 1) + E]) y -= tp[c * (E + 1) + E], --c;
+  if (c < 0) return;
+  const int* const tc = tp + c * (E + 1);
+  int lo = 0, hi = E - 1;            // expert e with tc[e] <= y < tc[e + 1]
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (tp[mid] <= y) lo = mid; else hi = mid - 1;
+    if (tc[mid] <= y) lo = mid; else hi = mid - 1;
   }
   const int e = lo;
   const int r0 = offsets[e], r1 = offsets[e + 1];
-  const int mb = r0 + (y - tp[e]) * BM;
+  // Full tiles come first in an expert; only class RB - 1 holds more than one.
+  const int mb = r0 + (c == RB - 1 ? y - tc[e] : (r1 - r0) / BM) * BM;
+  __syncthreads();                   // the prefixes have been read: the ring may start
   const int rows = min(BM, r1 - mb);
   const int half = N / 2;
   const int o0 = act ? bx * (BN / 2) : bx * BN;
@@ -724,16 +738,18 @@ int grouped_gemm(const uint16_t* X, const int32_t* sorted_idx, const int32_t* of
   do {                                                                                         \
     constexpr int BM = WM * 32 * RB, BN = WN * 64;                                             \
     const int gx = act ? mm_cdiv(nout, BN / 2) : mm_cdiv(N, BN);                               \
-    const long blocks = (long)gx * ((tk + BM - 1) / BM + std::min<long>(E, tk));               \
+    const long run = std::max<long>(1, tk / ((long)E * BM));                                   \
+    const long tiles = (tk + BM - 1) / BM + std::min<long>(E, tk);                             \
+    const long blocks = (long)gx * ((tiles + 8 * run - 1) / (8 * run) * (8 * run));            \
     MM_CHECK_ARG(blocks < (1L << 30), "mm_moe_grouped_gemm: T*k=%ld too large", tk);           \
     if (g % PF2_BK == 0)                                                                       \
       hipLaunchKernelGGL((k_moe_prefill<WM, WN, RB, true, ST>), dim3((unsigned)blocks), \
                          dim3(WM * WN * 64), 0, (hipStream_t)stream, (const f16*)X, sorted_idx, \
-                         offsets, gather, k, W, E, K, N, g, act, gx, (f16*)Y);  \
+                         offsets, gather, k, W, E, K, N, g, act, gx, (int)run, (f16*)Y);  \
     else                                                                                       \
       hipLaunchKernelGGL((k_moe_prefill<WM, WN, RB, false, ST>), dim3((unsigned)blocks),\
                          dim3(WM * WN * 64), 0, (hipStream_t)stream, (const f16*)X, sorted_idx, \
-                         offsets, gather, k, W, E, K, N, g, act, gx, (f16*)Y);  \
+                         offsets, gather, k, W, E, K, N, g, act, gx, (int)run, (f16*)Y);  \
   } while (0)
     if (cfg == 1)
       MM_LAUNCH_MOE_PF(1, 4, 2, MOE_PF_STAGES);    // 64 x 256, 4 waves
