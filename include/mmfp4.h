@@ -233,6 +233,15 @@ int mm_moe_router(const uint16_t* X, const uint16_t* W, const float* bias, int T
 int mm_softmax_topk(const void* logits, int logits_f32, int T, int E, int k, int renorm,
                     int64_t* ids, float* probs, void* stream);
 
+/* mm_moe_router / mm_softmax_topk with the probabilities written as fp16, each
+ * rounded once from its fp32 value (what the reference's router returns for an
+ * fp16 gate). */
+int mm_moe_router_p16(const uint16_t* X, const uint16_t* W, const float* bias, int T, int H, int E,
+                      int k, int renorm, int64_t* ids, uint16_t* probs, void* ws, size_t ws_bytes,
+                      void* stream);
+int mm_softmax_topk_p16(const void* logits, int logits_f32, int T, int E, int k, int renorm,
+                        int64_t* ids, uint16_t* probs, void* stream);
+
 /* Grouped expert GEMM over expert-sorted rows.  For expert e, rows
  * r in [offsets[e], offsets[e+1]) compute Y[r] = X[row(r)] . dequant(B[e], S[e]),
  * where row(r) = sorted_idx[r] / k when gather != 0 (rows of X are tokens)
@@ -272,6 +281,13 @@ int mm_moe_mlp_fp4(const uint16_t* X, const void* expert_ids, int ids_i64, const
                    const uint32_t* Bdn, const uint16_t* Sdn, int group_size, uint16_t* act_buf,
                    uint16_t* y_buf, int32_t* sort_buf, uint16_t* out, void* stream);
 
+/* mm_moe_mlp_fp4 with fp16 probabilities [T, k]. */
+int mm_moe_mlp_fp4_p16(const uint16_t* X, const void* expert_ids, int ids_i64,
+                       const uint16_t* probs, int T, int k, int E, int H, int I,
+                       const uint32_t* Bgu, const uint16_t* Sgu, const uint32_t* Bdn,
+                       const uint16_t* Sdn, int group_size, uint16_t* act_buf, uint16_t* y_buf,
+                       int32_t* sort_buf, uint16_t* out, void* stream);
+
 /* mm_moe_mlp_fp4 plus a shared expert that every token visits:
  *   out[t] = base[t] + sum_j probs[t, j] * y_routed(t, j) + shared_weight * y_shared(t)
  * with y_shared(t) = (silu(h[:I]) * h[I:]) . W_sdn, h = X[t] . W_sgu, W_sgu
@@ -291,6 +307,15 @@ int mm_moe_mlp_shared_fp4(const uint16_t* X, const void* expert_ids, int ids_i64
                           const uint32_t* Bsdn, const uint16_t* Ssdn, float shared_weight,
                           const uint16_t* base, int group_size, uint16_t* act_buf,
                           uint16_t* y_buf, int32_t* sort_buf, uint16_t* out, void* stream);
+
+/* mm_moe_mlp_shared_fp4 with fp16 probabilities [T, k]. */
+int mm_moe_mlp_shared_fp4_p16(const uint16_t* X, const void* expert_ids, int ids_i64,
+                              const uint16_t* probs, int T, int k, int E, int H, int I,
+                              const uint32_t* Bgu, const uint16_t* Sgu, const uint32_t* Bdn,
+                              const uint16_t* Sdn, const uint32_t* Bsgu, const uint16_t* Ssgu,
+                              const uint32_t* Bsdn, const uint16_t* Ssdn, float shared_weight,
+                              const uint16_t* base, int group_size, uint16_t* act_buf,
+                              uint16_t* y_buf, int32_t* sort_buf, uint16_t* out, void* stream);
 
 /* Shared + routed aggregation of one FP4 projection (no MLP):
  *   out[t] = X[t] . W_sh + sum_j probs[t, j] * (X[t] . W_routed[e(t, j)])

@@ -540,7 +540,9 @@ k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
   // < e (wave c scans class c).  A tile's time is about (2 + live blocks), a
   // launch has one to two rounds of tiles, and in expert order the CUs that got
   // a full tile last kept the launch going while the others were idle (CUs busy
-  // 63% of the launch, 82% of a dense one): MM_MOE_LPT.
+  // 63% of the launch, 82% of a dense one).  Qwen3-30B-A3B shapes with uneven
+// loads, mean of gate_up and down at T = 1024: 77.5 -> 70.7 us; T = 512, 2048 and
+// 4096 within 2%.
   if (wave < RB) {
     int* const t = tp + wave * (E + 1);
     int base = 0;
@@ -630,13 +632,28 @@ k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
 // base may be null.  Summed in fp32 in slot order; one block per token, 8
 // columns per thread.  nvalid (may be null): the sort's count of valid
 // assignments; slots placed at or past it (dropped ids) contribute nothing.
+// PT: fp32 or fp16 probabilities (fp16 ones are exact in fp32, so callers that
+// hold them need no conversion launch: 4 us each way).  The slots' rows are
+// loaded CMB_U at a time, and a wave loads its token's weights once, one per
+// lane.  T = 32, H = 2048, k = 8: 4.9 us one row at a time, 4.0 so (T = 1024 7.8,
+// 8.0).
+constexpr int CMB_U = 4;
+template <typename PT>
 __global__ void __launch_bounds__(256)
-k_moe_combine(const f16* __restrict__ Y, const float* __restrict__ probs,
+k_moe_combine(const f16* __restrict__ Y, const PT* __restrict__ probs,
               const int32_t* __restrict__ inverse, int k, int kin, float wsh,
               const f16* __restrict__ base, const int32_t* __restrict__ nvalid, int H,
               f16* __restrict__ out) {
   const int t = blockIdx.x;
   const int lim = nvalid ? *nvalid : 0x7fffffff;
+  // Lane l of every wave holds the weight of slot l (all lanes load: the column
+  // loop below may leave some idle); slots past 63 are loaded when used.
+  auto load_weight = [&](int j) { return j < kin ? (float)probs[(size_t)t * kin + j] : wsh; };
+  const int lane_w = __builtin_bit_cast(int, load_weight(threadIdx.x & 63));
+  auto weight = [&](int j) {
+    return j < 64 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(lane_w, j))
+                  : load_weight(j);
+  };
   for (int h8 = threadIdx.x; h8 < H / 8; h8 += 256) {
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (base) {
@@ -644,13 +661,22 @@ k_moe_combine(const f16* __restrict__ Y, const float* __restrict__ probs,
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = (float)b[i];
     }
-    for (int j = 0; j < k; ++j) {
-      const float p = j < kin ? probs[(size_t)t * kin + j] : wsh;
-      const int r = inverse[(size_t)t * k + j];
-      if (r >= lim) continue;
-      const f16x8 y = *(const f16x8*)(Y + (size_t)r * H + 8 * h8);
+    for (int j0 = 0; j0 < k; j0 += CMB_U) {
+      int r[CMB_U];
+      f16x8 y[CMB_U];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] += p * (float)y[i];
+      for (int u = 0; u < CMB_U; ++u) r[u] = inverse[(size_t)t * k + min(j0 + u, k - 1)];
+      // Unconditional loads (row 0 in place of a dropped one), so all are in flight.
+#pragma unroll
+      for (int u = 0; u < CMB_U; ++u)
+        y[u] = *(const f16x8*)(Y + (size_t)(r[u] < lim ? r[u] : 0) * H + 8 * h8);
+#pragma unroll
+      for (int u = 0; u < CMB_U; ++u)
+        if (j0 + u < k && r[u] < lim) {
+          const float p = weight(j0 + u);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc[i] += p * (float)y[u][i];
+        }
     }
     f16x8 o;
 #pragma unroll
@@ -795,13 +821,14 @@ int grouped_gemm(const uint16_t* X, const int32_t* sorted_idx, const int32_t* of
 }
 
 
-int combine(const uint16_t* Y, const float* probs, const int32_t* inverse, int T, int k, int kin,
+template <typename PT>
+int combine(const uint16_t* Y, const PT* probs, const int32_t* inverse, int T, int k, int kin,
             float wsh, const uint16_t* base, const int32_t* nvalid, int H, uint16_t* out,
             void* stream) {
   MM_CHECK_ARG(T >= 0 && k > 0 && H > 0, "mm_moe_combine: bad shape");
   MM_CHECK_ARG(H % 8 == 0, "mm_moe_combine: H=%d must be divisible by 8", H);
   if (T == 0) return 0;
-  hipLaunchKernelGGL(k_moe_combine, dim3(T), dim3(256), 0, (hipStream_t)stream, (const f16*)Y,
+  hipLaunchKernelGGL(k_moe_combine<PT>, dim3(T), dim3(256), 0, (hipStream_t)stream, (const f16*)Y,
                      probs, inverse, k, kin, wsh, (const f16*)base, nvalid, H, (f16*)out);
   MM_CHECK_LAUNCH("mm_moe_combine");
   return 0;
@@ -817,8 +844,8 @@ int combine(const uint16_t* Y, const float* probs, const int32_t* inverse, int T
 // token visits with weight wsh: its rows share the two grouped launches with
 // the routed experts' rows, and the combine adds it as slot k.  k may then be
 // 0 (the shared expert alone).  base (may be null) is added in the combine.
-template <typename IdT>
-int moe_mlp(const char* who, const uint16_t* X, const IdT* ids, const float* probs, int T, int k,
+template <typename IdT, typename PT>
+int moe_mlp(const char* who, const uint16_t* X, const IdT* ids, const PT* probs, int T, int k,
             int E, int H, int I, const uint32_t* Bgu, const uint16_t* Sgu, const uint32_t* Bdn,
             const uint16_t* Sdn, const uint32_t* Bsgu, const uint16_t* Ssgu, const uint32_t* Bsdn,
             const uint16_t* Ssdn, float wsh, const uint16_t* base, int g, uint16_t* act_buf,
@@ -909,11 +936,11 @@ extern "C" int mm_moe_combine(const uint16_t* Y, const float* probs, const int32
   return combine(Y, probs, inverse, T, k, k, 0.0f, nullptr, nullptr, H, out, stream);
 }
 
-extern "C" int mm_moe_mlp_fp4(const uint16_t* X, const void* expert_ids, int ids_i64,
-                              const float* probs, int T, int k, int E, int H, int I,
-                              const uint32_t* Bgu, const uint16_t* Sgu, const uint32_t* Bdn,
-                              const uint16_t* Sdn, int g, uint16_t* act_buf, uint16_t* y_buf,
-                              int32_t* sort_buf, uint16_t* out, void* stream) {
+template <typename PT>
+static int mlp_fp4(const uint16_t* X, const void* expert_ids, int ids_i64, const PT* probs, int T,
+                   int k, int E, int H, int I, const uint32_t* Bgu, const uint16_t* Sgu,
+                   const uint32_t* Bdn, const uint16_t* Sdn, int g, uint16_t* act_buf,
+                   uint16_t* y_buf, int32_t* sort_buf, uint16_t* out, void* stream) {
   const char* who = "mm_moe_mlp_fp4";
   if (ids_i64)
     return moe_mlp(who, X, (const int64_t*)expert_ids, probs, T, k, E, H, I, Bgu, Sgu, Bdn, Sdn,
@@ -924,15 +951,32 @@ extern "C" int mm_moe_mlp_fp4(const uint16_t* X, const void* expert_ids, int ids
                  out, stream);
 }
 
-extern "C" int mm_moe_mlp_shared_fp4(const uint16_t* X, const void* expert_ids, int ids_i64,
-                                     const float* probs, int T, int k, int E, int H, int I,
-                                     const uint32_t* Bgu, const uint16_t* Sgu,
-                                     const uint32_t* Bdn, const uint16_t* Sdn,
-                                     const uint32_t* Bsgu, const uint16_t* Ssgu,
-                                     const uint32_t* Bsdn, const uint16_t* Ssdn,
-                                     float shared_weight, const uint16_t* base, int g,
-                                     uint16_t* act_buf, uint16_t* y_buf, int32_t* sort_buf,
-                                     uint16_t* out, void* stream) {
+extern "C" int mm_moe_mlp_fp4(const uint16_t* X, const void* expert_ids, int ids_i64,
+                              const float* probs, int T, int k, int E, int H, int I,
+                              const uint32_t* Bgu, const uint16_t* Sgu, const uint32_t* Bdn,
+                              const uint16_t* Sdn, int g, uint16_t* act_buf, uint16_t* y_buf,
+                              int32_t* sort_buf, uint16_t* out, void* stream) {
+  return mlp_fp4(X, expert_ids, ids_i64, probs, T, k, E, H, I, Bgu, Sgu, Bdn, Sdn, g, act_buf,
+                 y_buf, sort_buf, out, stream);
+}
+
+extern "C" int mm_moe_mlp_fp4_p16(const uint16_t* X, const void* expert_ids, int ids_i64,
+                                  const uint16_t* probs, int T, int k, int E, int H, int I,
+                                  const uint32_t* Bgu, const uint16_t* Sgu, const uint32_t* Bdn,
+                                  const uint16_t* Sdn, int g, uint16_t* act_buf, uint16_t* y_buf,
+                                  int32_t* sort_buf, uint16_t* out, void* stream) {
+  return mlp_fp4(X, expert_ids, ids_i64, (const f16*)probs, T, k, E, H, I, Bgu, Sgu, Bdn, Sdn, g,
+                 act_buf, y_buf, sort_buf, out, stream);
+}
+
+template <typename PT>
+static int mlp_shared_fp4(const uint16_t* X, const void* expert_ids, int ids_i64, const PT* probs,
+                          int T, int k, int E, int H, int I, const uint32_t* Bgu,
+                          const uint16_t* Sgu, const uint32_t* Bdn, const uint16_t* Sdn,
+                          const uint32_t* Bsgu, const uint16_t* Ssgu, const uint32_t* Bsdn,
+                          const uint16_t* Ssdn, float shared_weight, const uint16_t* base, int g,
+                          uint16_t* act_buf, uint16_t* y_buf, int32_t* sort_buf, uint16_t* out,
+                          void* stream) {
   const char* who = "mm_moe_mlp_shared_fp4";
   MM_CHECK_ARG(Bsgu != nullptr, "%s: the shared expert's gate_up weights are required", who);
   if (ids_i64 || k == 0)
@@ -943,6 +987,24 @@ extern "C" int mm_moe_mlp_shared_fp4(const uint16_t* X, const void* expert_ids, 
                  Bsgu, Ssgu, Bsdn, Ssdn, shared_weight, base, g, act_buf, y_buf, sort_buf, out,
                  stream);
 }
+
+#define MM_SHARED_PARAMS(PT)                                                                      \
+  const uint16_t *X, const void *expert_ids, int ids_i64, const PT *probs, int T, int k, int E,     \
+      int H, int I, const uint32_t *Bgu, const uint16_t *Sgu, const uint32_t *Bdn,                  \
+      const uint16_t *Sdn, const uint32_t *Bsgu, const uint16_t *Ssgu, const uint32_t *Bsdn,        \
+      const uint16_t *Ssdn, float shared_weight, const uint16_t *base, int g, uint16_t *act_buf,    \
+      uint16_t *y_buf, int32_t *sort_buf, uint16_t *out, void *stream
+extern "C" int mm_moe_mlp_shared_fp4(MM_SHARED_PARAMS(float)) {
+  return mlp_shared_fp4(X, expert_ids, ids_i64, probs, T, k, E, H, I, Bgu, Sgu, Bdn, Sdn, Bsgu,
+                        Ssgu, Bsdn, Ssdn, shared_weight, base, g, act_buf, y_buf, sort_buf, out,
+                        stream);
+}
+extern "C" int mm_moe_mlp_shared_fp4_p16(MM_SHARED_PARAMS(uint16_t)) {
+  return mlp_shared_fp4(X, expert_ids, ids_i64, (const f16*)probs, T, k, E, H, I, Bgu, Sgu, Bdn,
+                        Sdn, Bsgu, Ssgu, Bsdn, Ssdn, shared_weight, base, g, act_buf, y_buf,
+                        sort_buf, out, stream);
+}
+#undef MM_SHARED_PARAMS
 
 extern "C" int mm_moe_gemm_shared_fp4(const uint16_t* X, const void* expert_ids, int ids_i64,
                                       const float* probs, int T, int k, int E, int K, int N,

@@ -66,6 +66,9 @@ SIGNATURES: dict[str, tuple] = {
     "mm_fp4_flat_dequantize": (_c_int, [_vp, _vp, _c_size, _c_size, _c_int, _vp, _vp]),
     "mm_fp4_pack_pair": (_c_int, [_vp, _vp, _c_size, _vp, _vp]),
 }
+# the same arguments with fp16 probabilities
+for _n in ("mm_moe_router", "mm_softmax_topk", "mm_moe_mlp_fp4", "mm_moe_mlp_shared_fp4"):
+    SIGNATURES[_n + "_p16"] = SIGNATURES[_n]
 
 _lib = None
 _lock = threading.Lock()

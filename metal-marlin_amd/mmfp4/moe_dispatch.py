@@ -121,11 +121,12 @@ _FUSED_ROUTER_MAX_WORK = 1 << 25        # T * H * E
 
 
 def _router(hidden: torch.Tensor, weight_eh: torch.Tensor, bias: torch.Tensor | None,
-            top_k: int, renormalize: bool):
+            top_k: int, renormalize: bool, dtype: torch.dtype = torch.float32):
     """logits = hidden @ weight_eh^T (+ bias), rounded to fp16 as the gate's
     fp16 output is, then fp32 softmax -> top-k -> optional renormalisation.
     Decode-sized T: one launch (`mm_moe_router`); larger T: the library GEMM
-    then `mm_softmax_topk`.  Returns (probs fp32 [T, k], ids int64 [T, k])."""
+    then `mm_softmax_topk`.  Returns (probs [T, k] in fp32, or in fp16 when dtype
+    says so, ids int64 [T, k])."""
     dev = _lib.require_device(hidden, weight_eh, bias)
     H = hidden.shape[-1]
     x = _half(hidden.reshape(-1, H))
@@ -135,13 +136,15 @@ def _router(hidden: torch.Tensor, weight_eh: torch.Tensor, bias: torch.Tensor | 
     if T > _FUSED_ROUTER_MAX_T or T * H * E > _FUSED_ROUTER_MAX_WORK:
         w16 = weight_eh.to(torch.float16).contiguous()
         b16 = None if bias is None else bias.to(torch.float16)
-        return _softmax_topk(torch.nn.functional.linear(x, w16, b16), top_k, renormalize)
+        return _softmax_topk(torch.nn.functional.linear(x, w16, b16), top_k, renormalize, dtype)
     w = _half(weight_eh)
     b = None if bias is None else bias.to(torch.float32).contiguous()
+    p16 = dtype == torch.float16
     ids = torch.empty((T, top_k), dtype=torch.int64, device=dev)
-    probs = torch.empty((T, top_k), dtype=torch.float32, device=dev)
+    probs = torch.empty((T, top_k), dtype=dtype if p16 else torch.float32, device=dev)
     ws = _lib.workspace(dev, int(_lib.load().mm_moe_router_workspace_bytes(T, H, E)))
-    _lib.call("mm_moe_router", _lib.ptr(x), _lib.ptr(w), _lib.ptr(b), T, H, E, top_k,
+    _lib.call("mm_moe_router_p16" if p16 else "mm_moe_router", _lib.ptr(x), _lib.ptr(w),
+              _lib.ptr(b), T, H, E, top_k,
               int(renormalize), _lib.ptr(ids), _lib.ptr(probs), _lib.ptr(ws), ws.numel(),
               _lib.stream_of(x))
     return probs, ids
@@ -164,21 +167,26 @@ def fused_router_topk(hidden_states: torch.Tensor, gate: nn.Linear, top_k: int,
     topk_indices int64).  `training` and `use_metal` are accepted for
     signature parity; there is one implementation."""
     probs, ids = _router(hidden_states, gate.weight.detach(),
-                         None if gate.bias is None else gate.bias.detach(), top_k, True)
+                         None if gate.bias is None else gate.bias.detach(), top_k, True,
+                         gate.weight.dtype)
     return probs.to(gate.weight.dtype), ids
 
 
-def _softmax_topk(gate_logits: torch.Tensor, top_k: int, renormalize: bool):
-    """mm_softmax_topk over logits [..., E] -> (probs fp32 [T, k], ids int64 [T, k])."""
+def _softmax_topk(gate_logits: torch.Tensor, top_k: int, renormalize: bool,
+                  dtype: torch.dtype = torch.float32):
+    """mm_softmax_topk over logits [..., E] -> (probs [T, k] in fp32, or in fp16
+    when dtype says so, ids int64 [T, k])."""
     dev = _lib.require_device(gate_logits)
     E = gate_logits.shape[-1]
     lg = gate_logits.reshape(-1, E)
     f32 = lg.dtype != torch.float16
     lg = (lg.to(torch.float32) if f32 else lg).contiguous()
     T = lg.shape[0]
+    p16 = dtype == torch.float16
     ids = torch.empty((T, top_k), dtype=torch.int64, device=dev)
-    probs = torch.empty((T, top_k), dtype=torch.float32, device=dev)
-    _lib.call("mm_softmax_topk", _lib.ptr(lg), int(f32), T, E, top_k, int(renormalize),
+    probs = torch.empty((T, top_k), dtype=dtype if p16 else torch.float32, device=dev)
+    _lib.call("mm_softmax_topk_p16" if p16 else "mm_softmax_topk", _lib.ptr(lg), int(f32), T, E,
+              top_k, int(renormalize),
               _lib.ptr(ids), _lib.ptr(probs), _lib.stream_of(lg))
     return probs, ids
 
@@ -188,7 +196,7 @@ def router_softmax_topk(gate_logits: torch.Tensor, top_k: int, renormalize: bool
     logits [T, E] in one launch (moe_dispatch.py:99-151,
     _router_softmax_fusion).  Returns (topk_probs in the logits' dtype,
     topk_indices int64)."""
-    probs, ids = _softmax_topk(gate_logits, top_k, renormalize)
+    probs, ids = _softmax_topk(gate_logits, top_k, renormalize, gate_logits.dtype)
     lead = tuple(gate_logits.shape[:-1])
     return probs.to(gate_logits.dtype).reshape(*lead, top_k), ids.reshape(*lead, top_k)
 
@@ -288,7 +296,8 @@ def moe_mlp_fp4(hidden: torch.Tensor, gate_up_packed: torch.Tensor, gate_up_scal
         raise ValueError(f"hidden size {x.shape[-1]} != packed K={H}")
     i64 = expert_ids.dtype == torch.int64
     ids = expert_ids.contiguous() if i64 else expert_ids.to(torch.int32).contiguous()
-    p = expert_probs.to(torch.float32).contiguous()
+    p16 = expert_probs.dtype == torch.float16
+    p = expert_probs.to(torch.float16 if p16 else torch.float32).contiguous()
     act = torch.empty((T * k, I), dtype=torch.float16, device=dev)
     y = torch.empty((T * k, H), dtype=torch.float16, device=dev)
     sort_buf = torch.empty(E + 1 + 2 * T * k, dtype=torch.int32, device=dev)
@@ -296,7 +305,8 @@ def moe_mlp_fp4(hidden: torch.Tensor, gate_up_packed: torch.Tensor, gate_up_scal
     # converted copies are bound to names so they outlive the launch
     gu, gus = gate_up_packed.contiguous(), _half(gate_up_scales)
     dn, dns = down_packed.contiguous(), _half(down_scales)
-    _lib.call("mm_moe_mlp_fp4", _lib.ptr(x), _lib.ptr(ids), int(i64), _lib.ptr(p), T, k, E, H, I,
+    _lib.call("mm_moe_mlp_fp4_p16" if p16 else "mm_moe_mlp_fp4", _lib.ptr(x), _lib.ptr(ids),
+              int(i64), _lib.ptr(p), T, k, E, H, I,
               _lib.ptr(gu), _lib.ptr(gus), _lib.ptr(dn), _lib.ptr(dns), group_size,
               _lib.ptr(act), _lib.ptr(y), _lib.ptr(sort_buf), _lib.ptr(out), _lib.stream_of(x))
     return out if hidden.dtype == torch.float16 else out.to(hidden.dtype)
@@ -380,6 +390,7 @@ def _moe_mlp_shared(hidden: torch.Tensor, routed, shared, expert_ids, expert_pro
             tuple(sdns.shape) != (I // group_size, H):
         raise ValueError("shared expert scales must be [H/g, 2I] and [I/g, H]")
     dev = _lib.require_device(x, sgu, sgus, sdn, sdns, expert_ids, expert_probs, base)
+    p16 = routed is not None and expert_probs.dtype == torch.float16
     if routed is None:
         k, E = 0, 0
         gu = gus = dn = dns = ids = p = None
@@ -398,7 +409,7 @@ def _moe_mlp_shared(hidden: torch.Tensor, routed, shared, expert_ids, expert_pro
         k = expert_ids.shape[1]
         i64 = int(expert_ids.dtype == torch.int64)
         ids = expert_ids.contiguous() if i64 else expert_ids.to(torch.int32).contiguous()
-        p = expert_probs.to(torch.float32).contiguous()
+        p = expert_probs.to(torch.float16 if p16 else torch.float32).contiguous()
         gu, dn = gu.contiguous(), dn.contiguous()
         gus, dns = _half(gus), _half(dns)
     kt = k + 1
@@ -408,7 +419,8 @@ def _moe_mlp_shared(hidden: torch.Tensor, routed, shared, expert_ids, expert_pro
     sort_buf = torch.empty(E + 2 + 2 * T * kt, dtype=torch.int32, device=dev)
     out = torch.empty((T, H), dtype=torch.float16, device=dev)
     sgus_h, sdns_h = _half(sgus), _half(sdns)   # bound: they must outlive the launch
-    _lib.call("mm_moe_mlp_shared_fp4", _lib.ptr(x), _lib.ptr(ids), i64, _lib.ptr(p), T, k, E, H,
+    _lib.call("mm_moe_mlp_shared_fp4_p16" if p16 else "mm_moe_mlp_shared_fp4", _lib.ptr(x),
+              _lib.ptr(ids), i64, _lib.ptr(p), T, k, E, H,
               I, _lib.ptr(gu), _lib.ptr(gus), _lib.ptr(dn), _lib.ptr(dns), _lib.ptr(sgu),
               _lib.ptr(sgus_h), _lib.ptr(sdn), _lib.ptr(sdns_h), float(shared_weight),
               _lib.ptr(b), group_size, _lib.ptr(act), _lib.ptr(y), _lib.ptr(sort_buf),

@@ -330,3 +330,19 @@ def test_moe_mlp_out_aliases_hidden(rng, T):
               _lib.ptr(dGU), _lib.ptr(dGS), _lib.ptr(dDP), _lib.ptr(dDS), g, _lib.ptr(act),
               _lib.ptr(y), _lib.ptr(sort_buf), _lib.ptr(xin), _lib.stream_of(xin))
     assert torch.equal(xin, want)
+
+
+@pytest.mark.parametrize("T,k,H", [(1, 1, 8), (3, 8, 40), (2, 64, 2008), (2, 70, 512), (5, 6, 4104)])
+def test_combine_widths(rng, T, k, H):
+    """Combine where the column loop leaves lanes idle (H / 8 not a multiple of
+    64), at and past 64 slots."""
+    import mmfp4
+    from mmfp4.moe_dispatch import MoEDispatchInfo
+    y = torch.from_numpy(rng.normal(0, 1, (T * k, H)).astype(np.float16)).cuda()
+    p = torch.from_numpy(rng.uniform(0, 1, (T, k)).astype(np.float32)).cuda()
+    inv = torch.from_numpy(rng.permutation(T * k).astype(np.int64)).cuda()
+    info = MoEDispatchInfo(inv, inv, inv, inv, T, k, 1, inv)
+    announce(f"combine T={T} k={k} H={H}")
+    out = mmfp4.scatter_expert_outputs(y, p, info)
+    ref = (y[inv].view(T, k, H).double() * p.double().unsqueeze(-1)).sum(1)
+    assert torch.allclose(out.double(), ref, rtol=1e-3, atol=k * 2e-4)

@@ -167,3 +167,32 @@ def test_fused_router_bias_and_layouts(rng, T, H, E, k):
     announce(f"fused router bias T={T} H={H} E={E} k={k}")
     wts, ids = mmfp4.fused_router_topk(to_dev(x), gate, k)
     _check_topk(ids, wts.float(), ref, k, True)
+
+
+@pytest.mark.parametrize("T,E,k,renorm", [(1, 8, 2, True), (5, 128, 8, True), (33, 256, 6, False),
+                                          (7, 600, 3, True), (3, 2000, 4, False)])
+def test_fp16_probabilities(rng, T, E, k, renorm):
+    """fp16 logits: the probabilities come back fp16, each its fp32 value rounded
+    once, on every top-k form; the expert MLP takes fp16 and fp32 probabilities
+    alike."""
+    import mmfp4
+    from mmfp4 import moe_dispatch as md
+    lg = torch.from_numpy(rng.normal(0, 1, (T, E)).astype(np.float16)).cuda()
+    p32, i32 = md._softmax_topk(lg, k, renorm)
+    p16, i16 = mmfp4.router_softmax_topk(lg, k, renorm)
+    assert p32.dtype == torch.float32 and p16.dtype == torch.float16
+    assert torch.equal(p32.half(), p16) and torch.equal(i32, i16)
+    if E > 256:
+        return
+    H, I, g = 128, 64, 32
+    gate = torch.nn.Linear(H, E, bias=True, device="cuda", dtype=torch.float16)
+    x = torch.from_numpy(rng.normal(0, 1, (T, H)).astype(np.float16)).cuda()
+    r32, j32 = md._router(x, gate.weight.detach(), gate.bias.detach(), k, True)
+    r16, j16 = mmfp4.fused_router_topk(x, gate, k)
+    assert torch.equal(r32.half(), r16) and torch.equal(j32, j16)
+    w = [mmfp4.quantize_fp4(torch.from_numpy(rng.normal(0, .02, (E * n, kk)).astype(np.float16))
+                            .cuda(), g) for n, kk in ((2 * I, H), (H, I))]
+    st = [t.reshape(t.shape[0], E, -1).transpose(0, 1).contiguous() for pair in w for t in pair]
+    p = p16.to(torch.float16)
+    assert torch.equal(mmfp4.moe_mlp_fp4(x, *st, i16, p, g),
+                       mmfp4.moe_mlp_fp4(x, *st, i16, p.float(), g))
