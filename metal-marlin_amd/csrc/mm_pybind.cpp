@@ -1,11 +1,14 @@
-// Python binding of the per-call hot path (marlin_gemm_fp4 / marlin_gemm_int4)
-// for callers that issue one GEMM per Python call.  It does in C++ what the
+// Python binding of the per-call hot path (marlin_gemm_fp4 / marlin_gemm_int4,
+// the fused QKV and gate/up projections and the row-packed product) for callers
+// that issue one projection per Python call.  It does in C++ what the
 // ctypes path does in Python -- shape checks, the output allocation, the
 // per-(device, stream) workspace -- and calls the same C ABI entry points of
 // libmmfp4.so (mm_fp4_gemm / mm_u4_gemm).  torch is used only for tensor
 // arguments and the output allocation; the stream comes from the caller.
 #include <torch/extension.h>
 
+#include <algorithm>
+#include <array>
 #include <map>
 #include <mutex>
 #include <sstream>
@@ -134,6 +137,101 @@ at::Tensor gemm(const at::Tensor& A, const at::Tensor& B, const at::Tensor& S,
   return out;
 }
 
+// The fused projections below take the plain form of their operands only --
+// contiguous fp16 activations and scales and packed words on one device, shapes
+// that agree -- and return None for anything else, which their Python callers
+// then convert or refuse.
+bool plain(const at::Tensor& t, at::ScalarType type, int dev, int64_t d0, int64_t d1) {
+  return t.dim() == 2 && t.size(0) == d0 && t.size(1) == d1 && t.get_device() == dev &&
+         t.is_contiguous() && t.scalar_type() == type;
+}
+bool plain_words(const at::Tensor& t, int dev, int64_t d0, int64_t d1) {
+  return plain(t, t.scalar_type() == at::kUInt32 ? at::kUInt32 : at::kInt, dev, d0, d1);
+}
+// [M, K] of the activations, or M = -1.
+std::pair<int64_t, int64_t> plain_acts(const at::Tensor& A) {
+  if (A.dim() != 2 || A.get_device() < 0 || !A.is_contiguous() || A.scalar_type() != at::kHalf ||
+      A.size(0) == 0 || A.size(1) == 0)
+    return {-1, 0};
+  return {A.size(0), A.size(1)};
+}
+
+// Q, K, V = A . dequant(W[p], S[p]) in one mm_fp4_gemm_multi call.
+pybind11::object qkv(const at::Tensor& A, const std::array<at::Tensor, 3>& W,
+                     const std::array<at::Tensor, 3>& S, int64_t g, int64_t stream) {
+  const auto [M, K] = plain_acts(A);
+  if (M < 0 || g <= 0 || K % g != 0 || K % 8 != 0) return pybind11::none();
+  const int dev = (int)A.get_device();
+  const uint32_t* b[3];
+  const uint16_t* s[3];
+  uint16_t* c[3];
+  int n[3];
+  int64_t ntot = 0;
+  for (int p = 0; p < 3; ++p) {
+    const int64_t N = W[p].dim() == 2 ? W[p].size(1) : 0;
+    if (N <= 0 || N % 4 != 0 || !plain_words(W[p], dev, K / 8, N) ||
+        !plain(S[p], at::kHalf, dev, K / g, N))
+      return pybind11::none();
+    n[p] = (int)N;
+    ntot += N;
+  }
+  at::Tensor out[3];
+  size_t need = mm_gemm_workspace_bytes((int)M, (int)ntot, (int)K);
+  for (int p = 0; p < 3; ++p) {
+    out[p] = at::empty({M, n[p]}, A.options());
+    need = std::max(need, mm_gemm_workspace_bytes((int)M, n[p], (int)K));
+    b[p] = (const uint32_t*)W[p].data_ptr();
+    s[p] = (const uint16_t*)S[p].data_ptr();
+    c[p] = (uint16_t*)out[p].data_ptr();
+  }
+  at::Tensor ws = workspace(A, stream, need);
+  const int rc = mm_fp4_gemm_multi((const uint16_t*)A.data_ptr(), 3, b, s, c, n, (int)M, (int)K,
+                                   (int)g, ws.data_ptr(), (size_t)ws.numel(), (void*)stream);
+  if (rc) fail(rc);
+  return pybind11::make_tuple(out[0], out[1], out[2]);
+}
+
+// The gate/up pair: Marlin [K/8, N] words, or row-packed [N, K/8] ones.
+pybind11::object gate_up(const at::Tensor& A, const at::Tensor& Wg, const at::Tensor& Sg,
+                         const at::Tensor& Wu, const at::Tensor& Su, int64_t g, bool rows,
+                         bool act, int64_t stream) {
+  const auto [M, K] = plain_acts(A);
+  if (M < 0 || g <= 0 || K % g != 0 || K % 8 != 0 || Wg.dim() != 2) return pybind11::none();
+  const int dev = (int)A.get_device();
+  const int64_t N = Wg.size(rows ? 0 : 1), d0 = rows ? N : K / 8, d1 = rows ? K / 8 : N;
+  if (N <= 0 || N % 8 != 0 || !plain_words(Wg, dev, d0, d1) || !plain_words(Wu, dev, d0, d1) ||
+      !plain(Sg, at::kHalf, dev, K / g, N) || !plain(Su, at::kHalf, dev, K / g, N))
+    return pybind11::none();
+  at::Tensor out = at::empty({M, act ? N : 2 * N}, A.options());
+  at::Tensor ws = workspace(A, stream, mm_gemm_workspace_bytes((int)M, (int)(2 * N), (int)K));
+  const auto fn = rows ? mm_fp4_gate_up_rowpacked : mm_fp4_gate_up;
+  const int rc = fn((const uint16_t*)A.data_ptr(), (const uint32_t*)Wg.data_ptr(),
+                    (const uint16_t*)Sg.data_ptr(), (const uint32_t*)Wu.data_ptr(),
+                    (const uint16_t*)Su.data_ptr(), (uint16_t*)out.data_ptr(), (int)M, (int)N,
+                    (int)K, (int)g, act, ws.data_ptr(), (size_t)ws.numel(), (void*)stream);
+  if (rc) fail(rc);
+  return pybind11::cast(out);
+}
+
+// Row-packed product: W [N, K/8], scales [K/g, N].
+pybind11::object rowpacked(const at::Tensor& A, const at::Tensor& W, const at::Tensor& S,
+                           int64_t g, int64_t stream) {
+  const auto [M, K] = plain_acts(A);
+  if (M < 0 || g <= 0 || K % g != 0 || K % 8 != 0 || W.dim() != 2) return pybind11::none();
+  const int dev = (int)A.get_device();
+  const int64_t N = W.size(0);
+  if (N <= 0 || !plain_words(W, dev, N, K / 8) || !plain(S, at::kHalf, dev, K / g, N))
+    return pybind11::none();
+  at::Tensor out = at::empty({M, N}, A.options());
+  at::Tensor ws = workspace(A, stream, mm_gemm_workspace_bytes((int)M, (int)N, (int)K));
+  const int rc = mm_fp4_gemm_rowpacked(
+      (const uint16_t*)A.data_ptr(), (const uint32_t*)W.data_ptr(), (const uint16_t*)S.data_ptr(),
+      (uint16_t*)out.data_ptr(), (int)M, (int)N, (int)K, (int)g, 0, ws.data_ptr(),
+      (size_t)ws.numel(), (void*)stream);
+  if (rc) fail(rc);
+  return pybind11::cast(out);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -141,6 +239,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm", &gemm, "C = A . dequant(B, S[, Z]) on the given stream", pybind11::arg("A"),
         pybind11::arg("B"), pybind11::arg("S"), pybind11::arg("Z"), pybind11::arg("SZ"),
         pybind11::arg("group_size"), pybind11::arg("stream"));
+  m.def("qkv", &qkv, "mm_fp4_gemm_multi on plain operands, else None");
+  m.def("gate_up", &gate_up, "mm_fp4_gate_up[_rowpacked] on plain operands, else None");
+  m.def("rowpacked", &rowpacked, "mm_fp4_gemm_rowpacked on plain operands, else None");
   m.def("workspace", &workspace_for,
         "the zero-initialised workspace of (device index, raw stream), at least nbytes",
         pybind11::arg("device"), pybind11::arg("stream"), pybind11::arg("nbytes"));

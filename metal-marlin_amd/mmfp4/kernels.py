@@ -90,6 +90,24 @@ def _gemm(kind: str, A: torch.Tensor, B_packed: torch.Tensor, scales: torch.Tens
     return _gemm_ctypes(kind, A, B_packed, scales, zeros, group_size, sz)
 
 
+def _fast(name: str, *args):
+    """The per-call binding's entry `name` on the current stream: its result, or
+    None when the binding is absent or the operands are not in the plain form it
+    takes (the caller then converts or refuses them)."""
+    fast = _BINDING if _BINDING is not None else _binding()
+    if not fast:
+        return None
+    idx = args[0].get_device()
+    if idx < 0:
+        return None
+    try:
+        return getattr(fast, name)(*args, _lib.raw_stream(idx))
+    except RuntimeError as e:
+        if type(e) is RuntimeError:
+            raise _lib.MMError(str(e)) from None
+        raise
+
+
 def _sz_ok(scales: torch.Tensor, zeros: torch.Tensor | None) -> bool:
     return (zeros is not None and scales.dim() == 2 and zeros.shape == scales.shape
             and scales.shape[-1] % 4 == 0 and scales.is_cuda and zeros.device == scales.device)
@@ -196,6 +214,11 @@ def mmfp4_gemm_rowpacked(A: torch.Tensor, B_rows: torch.Tensor, scales: torch.Te
     runs the decode kernels; larger M the pipelined prefill kernel, which
     reads the words in place too but takes [K/group_size, N] scales (the
     other layout is transposed here, K/group_size x N halves)."""
+    if isinstance(A, torch.Tensor) and A.dim() == 2 and B_rows.dim() == 2 and \
+            scales.dim() == 2 and scales.shape[1] == B_rows.shape[0]:
+        out = _fast("rowpacked", A, B_rows, scales, group_size)
+        if out is not None:
+            return out
     dev = _lib.require_device(A, B_rows, scales)
     M, K = A.shape
     N, K_packed = B_rows.shape
@@ -242,6 +265,12 @@ def _gate_up(x: torch.Tensor, gate_packed: torch.Tensor, gate_scales: torch.Tens
              act: int) -> torch.Tensor:
     """One launch over the gate and up matrices, both Marlin [K/8, N]:
     act=1 -> silu(x @ Wg) * (x @ Wu) [M, N]; act=0 -> [x @ Wg | x @ Wu] [M, 2N]."""
+    if isinstance(x, torch.Tensor) and x.dim() == 2 and \
+            (x.shape[0] <= 32 or x.shape[1] % 64 == 0):
+        out = _fast("gate_up", x, gate_packed, gate_scales, up_packed, up_scales, group_size,
+                    False, bool(act))
+        if out is not None:
+            return out
     dev = _lib.require_device(x, gate_packed, gate_scales, up_packed, up_scales)
     if x.dim() != 2:
         raise ValueError(f"x must be 2D [M, K], got shape={tuple(x.shape)}")
@@ -323,6 +352,10 @@ def mmfp4_fused_gate_up(x: torch.Tensor, gate_packed: torch.Tensor, gate_scales:
     M = x.shape[0]
     if rowpacked_gemm_supported(M, N, K, group_size) and N % 8 == 0:
         # the row-packed words are read in place, no transpose
+        out = _fast("gate_up", x, gate_packed, gate_scales, up_packed, up_scales, group_size,
+                    True, True)
+        if out is not None:
+            return out
         dev = _lib.require_device(x, gate_packed, gate_scales, up_packed, up_scales)
         a = _half(x)
         out = torch.empty((M, N), dtype=torch.float16, device=dev)
@@ -355,6 +388,11 @@ def mmfp4_fused_qkv(A: torch.Tensor, Q_packed: torch.Tensor, Q_scales: torch.Ten
     and mid-sized M run one launch over all three matrices' column tiles;
     larger M one launch per matrix (the reference falls back to separate GEMMs
     for M > 1)."""
+    if isinstance(A, torch.Tensor) and A.dim() == 2:
+        out = _fast("qkv", A, (Q_packed, K_packed, V_packed), (Q_scales, K_scales, V_scales),
+                    group_size)
+        if out is not None:
+            return out
     dev = _lib.require_device(A, Q_packed, Q_scales, K_packed, K_scales, V_packed, V_scales)
     orig_shape = A.shape
     if A.dim() == 1:

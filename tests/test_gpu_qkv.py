@@ -65,3 +65,34 @@ def test_fused_qkv_errors():
     s = torch.zeros((1, 16), dtype=torch.float16, device="cuda")
     with pytest.raises(ValueError, match="K weights: K mismatch"):
         mmfp4.mmfp4_fused_qkv(x, p, s, p[:4], s, p, s, 64)
+
+
+@pytest.mark.parametrize("M", [1, 40])
+def test_binding_and_ctypes_agree(monkeypatch, M):
+    """The fused projections and the row-packed product through the per-call
+    binding and through ctypes: same results, and operands that are not in the
+    binding's plain form (strided, other types) give them too."""
+    import mmfp4
+    from mmfp4 import kernels
+    K, N, g = 256, 72, 64
+    gen = torch.Generator("cuda").manual_seed(3)
+    w = torch.randn(3, N, K, device="cuda", generator=gen) * 0.02
+    marlin = [t for i in range(3) for t in mmfp4.quantize_fp4(w[i], g)]
+    rows = [t.t().contiguous() if i % 2 == 0 else t for i, t in enumerate(marlin)]
+    x = torch.randn(M, K, device="cuda", generator=gen).half()
+    odd = [marlin[0].t().contiguous().t(), marlin[1].float()] + marlin[2:]
+
+    def calls():
+        yield from mmfp4.mmfp4_fused_qkv(x, *marlin, g)
+        yield from mmfp4.mmfp4_fused_qkv(x.float(), *odd, g)
+        yield mmfp4.mmfp4_fused_gate_up_marlin(x, *marlin[:4], g)
+        yield mmfp4.fused_gate_up_gemm(x, *odd[:4], g)
+        yield mmfp4.mmfp4_fused_gate_up(x, *rows[:4], g)
+        yield mmfp4.mmfp4_gemm_rowpacked(x, rows[0], rows[1], g)
+        yield mmfp4.mmfp4_gemm_rowpacked(x, rows[0], rows[1].t().contiguous(), g)
+
+    announce(f"binding against ctypes M={M}")
+    fast = list(calls())
+    monkeypatch.setattr(kernels, "_BINDING", False)
+    for a, b in zip(fast, calls(), strict=True):
+        assert a.shape == b.shape and torch.equal(a, b)
