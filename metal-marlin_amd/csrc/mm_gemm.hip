@@ -277,12 +277,13 @@ k_skinny(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
 // grid of narrow layers without a K split.
 // ROWP: row-packed FP4 words [N, K/8] (K % 512 == 0), transposed through
 // LDS into the Marlin operand order (skinny_wave RT); scales [N, K/g] when
-// SROW, else [K/g, N].
-template <int INT4, int SPW, int NW, int FL, bool SROW = false, bool ROWP = false>
+// SROW, else [K/g, N].  MULTI: the tiles of up to three matrices in turn (mp).
+template <int INT4, int SPW, int NW, int FL, bool SROW = false, bool ROWP = false,
+          bool MULTI = false>
 __global__ void __launch_bounds__(NW * 64)
 k_skinny_dual(const f16* __restrict__ A, const uint32_t* __restrict__ B,
               const f16* __restrict__ S, const f16* __restrict__ Z, f16* __restrict__ C, int M,
-              int N, int K, int g, int nrounds) {
+              int N, int K, int g, int nrounds, SkMulti mp) {
   // ROWP: each wave stages its weights through 8 KiB of LDS in the main
   // loop; the block reduction reuses the same memory afterwards.
   constexpr int RED = row_items_lds_floats<1, 1, NW>();
@@ -290,7 +291,16 @@ k_skinny_dual(const f16* __restrict__ A, const uint32_t* __restrict__ B,
   __shared__ __attribute__((aligned(16))) float red[LDSF];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, q = lane >> 4;
-  const int n0 = blockIdx.x * 32;
+  int tile = blockIdx.x;
+  if constexpr (MULTI) {
+    const int p = tile >= mp.tile0[2] ? 2 : (tile >= mp.tile0[1] ? 1 : 0);
+    B = mp.B[p];
+    S = mp.S[p];
+    C = mp.C[p];
+    N = mp.N[p];
+    tile -= mp.tile0[p];
+  }
+  const int n0 = tile * 32;
   f32x4 acc[1][1][4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[0][0][j] = f32x4{0, 0, 0, 0};
@@ -980,6 +990,7 @@ int launch_skinny_nt2(const f16* A, const uint32_t* B, const f16* S, const f16* 
 #define MM_SK_DUAL_MIN_TILES 96
 #endif
 
+// N: columns of the product, or of all the products of a multi launch.
 bool use_dual(int M, int N, int K, int g) {
   if (M > 8 || K % 64 != 0 || g % 64 != 0 || N % 4 != 0) return false;
   if (flush_steps(g / 2, MM_SK_DUAL_SPW) == 0) return false;
@@ -987,16 +998,25 @@ bool use_dual(int M, int N, int K, int g) {
          mm_cdiv(N, SK_COLS) < MM_SK_DUAL_BELOW && mm_cdiv(N, 32) >= MM_SK_DUAL_MIN_TILES;
 }
 
-template <int INT4, bool SROW = false>
+template <int INT4, bool SROW = false, bool MULTI = false>
 int launch_dual(const f16* A, const uint32_t* B, const f16* S, const f16* Z, f16* C, int M, int N,
-                int K, int g, hipStream_t st) {
+                int K, int g, hipStream_t st, SkMulti* mp = nullptr) {
   constexpr int SPW = MM_SK_DUAL_SPW, NW = MM_SK_DUAL_NW;
   const int nsteps = K / 64;                           // 64-k steps
   const int nrounds = mm_cdiv(nsteps, NW * SPW);
   const int fl = flush_steps(g / 2, SPW);              // 64-k steps per scale group
+  int tiles = mm_cdiv(N, 32);
+  if (MULTI) {
+    tiles = 0;
+    for (int i = 0; i < 3; ++i) {
+      mp->tile0[i] = tiles;
+      tiles += mm_cdiv(mp->N[i], 32);
+    }
+  }
+  const SkMulti none{};
 #define MM_LAUNCH_DU(FLV)                                                                      \
-  hipLaunchKernelGGL((k_skinny_dual<INT4, SPW, NW, FLV, SROW>), dim3(mm_cdiv(N, 32)), dim3(NW * 64), 0, \
-                     st, A, B, S, Z, C, M, N, K, g, nrounds)
+  hipLaunchKernelGGL((k_skinny_dual<INT4, SPW, NW, FLV, SROW, false, MULTI>), dim3(tiles),       \
+                     dim3(NW * 64), 0, st, A, B, S, Z, C, M, N, K, g, nrounds, MULTI ? *mp : none)
   switch (fl) {
     case 1: MM_LAUNCH_DU(1); break;
     case 2: MM_LAUNCH_DU(2); break;
@@ -1462,6 +1482,10 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
   MM_CHECK_ARG((al & 15) == 0, "%s: A, B 16-byte / scales, C 8-byte alignment required", who);
   MM_CHECK_ARG(tiles <= SK_MAX_TILES, "%s: too many columns", who);
   if (M == 0) return 0;
+  // Two-slab kernel where one product of the same width takes it.
+  if (use_dual(M, ntot, K, g))
+    return launch_dual<false, false, true>(A, nullptr, nullptr, nullptr, nullptr, M, ntot, K, g,
+                                           st, &mp);
   if (M > 16)
     return launch_skinny<false, 2, SK_MULTI>(A, K, nullptr, nullptr, nullptr, nullptr, nullptr,
                                              nullptr, nullptr, 0, M, ntot, K, g, ws, ws_bytes, st,
@@ -1567,7 +1591,7 @@ extern "C" int mm_fp4_gemm_rowpacked(const uint16_t* A, const uint32_t* B, const
 #define MM_LAUNCH_RDU(FLV, SR)                                                                  \
   hipLaunchKernelGGL((k_skinny_dual<false, 8, NW, FLV, SR, true>), dim3(mm_cdiv(N, 32)),       \
                      dim3(NW * 64), 0, st, (const f16*)A, B, (const f16*)S, nullptr, (f16*)C, M,  \
-                     N, K, g, nr)
+                     N, K, g, nr, SkMulti{})
 #define MM_LAUNCH_RDU_FL(SR)                                                                    \
   switch (fl) {                                                                                \
     case 1: MM_LAUNCH_RDU(1, SR); break;                                                       \

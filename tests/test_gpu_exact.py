@@ -337,3 +337,17 @@ def test_multi_qkv_two_row_blocks(rng, M):
     announce(f"qkv two row blocks M={M}")
     for o, (p, s) in zip(mmfp4.mmfp4_fused_qkv(a, *args, g), w):
         _same(o, ofp4.gemm_fp4_ref(to_np(a), p, s, g))
+
+
+@pytest.mark.parametrize("M,K,Ns", [(1, 4096, (4096, 1024, 1024)), (8, 2048, (3004, 36, 64)),
+                                    (5, 4160, (2048, 1028, 4))])
+def test_multi_qkv_two_slab(rng, M, K, Ns):
+    """The two-slab kernel over three matrices, widths that end inside a tile."""
+    import mmfp4
+    g = 64
+    w = [_exact_fp4(rng, K, n, g) for n in Ns]
+    a = to_dev(_acts(rng, M, K))
+    announce(f"qkv two-slab M={M} K={K} {Ns}")
+    out = mmfp4.mmfp4_fused_qkv(a, *[to_dev(t) for pair in w for t in pair], g)
+    for o, (p, s) in zip(out, w):
+        _same(o, ofp4.gemm_fp4_ref(to_np(a), p, s, g))
