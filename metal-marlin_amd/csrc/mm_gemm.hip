@@ -664,7 +664,8 @@ k_prefill2(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
 // an arrival counter per tile, the last block adds the splits in split order):
 // a separate reduction launch costs about 5 us, a quarter of these calls.
 // ===========================================================================
-template <bool INT4, int RB, int WN, bool G128, int ACT>
+// ROWS: B (and B2) are row-packed [N, K/8] FP4 words.
+template <bool INT4, int RB, int WN, bool G128, int ACT, bool ROWS = false>
 __global__ void __launch_bounds__(WN * 256, RB <= 2 ? 4 : 2)
 k_mid(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
       const f16* __restrict__ S, const f16* __restrict__ Z, const uint32_t* __restrict__ B2,
@@ -690,7 +691,13 @@ k_mid(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
   const int m0 = blockIdx.y * Sh::BM, n0 = bx * (PAIR ? Sh::BN / 2 : Sh::BN);
   const int c_beg = blockIdx.z * cps, c_end = min(K / mmmid::MID_BK, c_beg + cps);
   f32x16 acc[RB][2];
-  if constexpr (PAIR) {
+  if constexpr (ROWS && PAIR) {
+    const PairRowSrc src{A, lda, M, m0, N, n0, B, B2, S, S2, Z, Z2, N, K / 8};
+    mmmid::mid_mainloop<INT4, RB, WN, G128, true>(src, K, g, c_beg, c_end, smem, acc);
+  } else if constexpr (ROWS) {
+    const DenseRowSrc src{A, lda, M, m0, N, n0, B, S, Z, N, K / 8};
+    mmmid::mid_mainloop<INT4, RB, WN, G128, false>(src, K, g, c_beg, c_end, smem, acc);
+  } else if constexpr (PAIR) {
     const PairSrc src{A, lda, M, m0, N, n0, B, B2, S, S2, Z, Z2, N};
     mmmid::mid_mainloop<INT4, RB, WN, G128, true>(src, K, g, c_beg, c_end, smem, acc);
   } else {
@@ -1136,6 +1143,8 @@ size_t prefill_ws_bytes(int M, int N, int K) {
 //   M = 100: 4096 -> 2 x 14336 43.1 -> 35.6, 4096 -> 4096 20.9 -> 13.1,
 //            14336 -> 4096 28.0 -> 24.1
 //   M = 512: 4096 -> 4096 31.8 -> 22.1; INT4 4096 -> 6144 59.6 -> 50.5
+//   row-packed M = 100: 4096 -> 2 x 14336 44.2 -> 35.2, 14336 -> 4096 28.0 -> 22.3;
+//            M = 300 122.8 -> 93.6 and 67.4 -> 52.8
 // What bounds it is LDS traffic and the matrix cores together.  Its time grows
 // smoothly with the tile count, the prefill tiles' in rounds of 256, so above
 // 128 rows the two are compared (mid_us, prefill_us): M = 512, 4096 -> 6144
@@ -1180,7 +1189,7 @@ size_t mid_ws_bytes(int M, int N, int K) {
   return need;
 }
 
-template <bool INT4, int ACT, int RB, int WN>
+template <bool INT4, int ACT, int RB, int WN, bool ROWS>
 int launch_mid_tile(const f16* A, const uint32_t* B, const f16* S, const f16* Z,
                     const uint32_t* B2, const f16* S2, const f16* Z2, f16* C, int ldc, int M,
                     int N, int K, int g, const MidPlan& p, int gx, void* ws, size_t ws_bytes,
@@ -1197,10 +1206,10 @@ int launch_mid_tile(const f16* A, const uint32_t* B, const f16* S, const f16* Z,
   }
   const SkMulti none{};
   if (g % 128 == 0)
-    hipLaunchKernelGGL((k_mid<INT4, RB, WN, true, ACT>), grid, dim3(Sh::NTHR), 0, st, A, K, B, S,
+    hipLaunchKernelGGL((k_mid<INT4, RB, WN, true, ACT, ROWS>), grid, dim3(Sh::NTHR), 0, st, A, K, B, S,
                        Z, B2, S2, Z2, C, ldc, M, N, K, g, p.cps, part, counters, mp ? *mp : none);
   else
-    hipLaunchKernelGGL((k_mid<INT4, RB, WN, false, ACT>), grid, dim3(Sh::NTHR), 0, st, A, K, B, S,
+    hipLaunchKernelGGL((k_mid<INT4, RB, WN, false, ACT, ROWS>), grid, dim3(Sh::NTHR), 0, st, A, K, B, S,
                        Z, B2, S2, Z2, C, ldc, M, N, K, g, p.cps, part, counters, mp ? *mp : none);
   MM_CHECK_LAUNCH("gemm(mid)");
   return 0;
@@ -1215,7 +1224,7 @@ bool mid_ok(const f16* S, const f16* Z, int N, int g) {
 
 // Column tiles per matrix: PLAIN / MULTI 64 * wn columns, pair forms 32 * wn of
 // each.  A K split has at most 256 tiles (plan_mid_tiles), so its counters fit.
-template <bool INT4, int ACT>
+template <bool INT4, int ACT, bool ROWS = false>
 int launch_mid(const MidPlan& p, const f16* A, const uint32_t* B, const f16* S, const f16* Z,
                const uint32_t* B2, const f16* S2, const f16* Z2, f16* C, int ldc, int M, int N,
                int K, int g, void* ws, size_t ws_bytes, hipStream_t st, SkMulti* mp = nullptr) {
@@ -1230,8 +1239,8 @@ int launch_mid(const MidPlan& p, const f16* A, const uint32_t* B, const f16* S, 
     mp->tile0[3] = gx;
   }
 #define MM_LAUNCH_MID(RBV, WNV)                                                                 \
-  return launch_mid_tile<INT4, ACT, RBV, WNV>(A, B, S, Z, B2, S2, Z2, C, ldc, M, N, K, g, p, gx, ws, \
-                                              ws_bytes, st, mp)
+  return launch_mid_tile<INT4, ACT, RBV, WNV, ROWS>(A, B, S, Z, B2, S2, Z2, C, ldc, M, N, K, g, p, \
+                                                    gx, ws, ws_bytes, st, mp)
   if (p.rb == 4) MM_LAUNCH_MID(4, 2);
   if (p.wn == 1) MM_LAUNCH_MID(2, 1);
   MM_LAUNCH_MID(2, 2);
@@ -1482,7 +1491,9 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
   MM_CHECK_ARG((al & 15) == 0, "%s: A, B 16-byte / scales, C 8-byte alignment required", who);
   MM_CHECK_ARG(tiles <= SK_MAX_TILES, "%s: too many columns", who);
   if (M == 0) return 0;
-  // Two-slab kernel where one product of the same width takes it.
+  // Two-slab kernel where one product of the same width takes it (4096 ->
+  // 4096 + 1024 + 1024 at M = 1: 7.1 -> 6.1 us of the layer's call against the
+  // 64-column tiles and their split-K hand-off).
   if (use_dual(M, ntot, K, g))
     return launch_dual<false, false, true>(A, nullptr, nullptr, nullptr, nullptr, M, ntot, K, g,
                                            st, &mp);
@@ -1553,7 +1564,12 @@ extern "C" int mm_fp4_gemm_rowpacked(const uint16_t* A, const uint32_t* B, const
                                                 g, ws, ws_bytes, st);
   }
   if (M > 32) {
-    // Pipelined prefill kernel reading the row-packed words in place.
+    // Mid and prefill kernels reading the row-packed words in place.
+    if (const MidPlan mid = plan_mid(M, N, K);
+        mid.wn != 0 && mid_ok<false>((const f16*)S, nullptr, N, g))
+      return launch_mid<false, SK_PLAIN, true>(mid, (const f16*)A, B, (const f16*)S, nullptr,
+                                               nullptr, nullptr, nullptr, (f16*)C, N, M, N, K, g,
+                                               ws, ws_bytes, st);
     const PrefillPlan p = plan_prefill(M, N, K);
     float* part = nullptr;
     if (p.ksplit > 1) {
@@ -1677,8 +1693,18 @@ extern "C" int mm_fp4_gate_up_rowpacked(const uint16_t* A, const uint32_t* Bg, c
                                                ws, ws_bytes, (hipStream_t)stream);
   }
   if (M > 32) {
-    // Pipelined prefill kernel reading both row-packed matrices in place;
-    // split and workspace as the unfused [K, 2N] product.
+    // Mid and prefill kernels reading both row-packed matrices in place; split
+    // and workspace as the unfused [K, 2N] product.
+    const f16 *a = (const f16*)A, *sg = (const f16*)Sg, *su = (const f16*)Su;
+    hipStream_t st = (hipStream_t)stream;
+    if (const MidPlan mid = plan_mid(M, 2 * N, K);
+        mid.wn != 0 && mid_ok<false>(sg, nullptr, N, g) && mid_ok<false>(su, nullptr, N, g)) {
+      if (act)
+        return launch_mid<false, SK_SWIGLU, true>(mid, a, Bg, sg, nullptr, Bu, su, nullptr,
+                                                  (f16*)C, ldc, M, N, K, g, ws, ws_bytes, st);
+      return launch_mid<false, SK_PAIR, true>(mid, a, Bg, sg, nullptr, Bu, su, nullptr, (f16*)C,
+                                              ldc, M, N, K, g, ws, ws_bytes, st);
+    }
     const PrefillPlan p = plan_prefill(M, 2 * N, K);
     float* part = nullptr;
     if (p.ksplit > 1) {
@@ -1688,8 +1714,6 @@ extern "C" int mm_fp4_gate_up_rowpacked(const uint16_t* A, const uint32_t* Bg, c
                    need);
       part = (float*)((char*)ws + SK_COUNTER_BYTES);
     }
-    const f16 *a = (const f16*)A, *sg = (const f16*)Sg, *su = (const f16*)Su;
-    hipStream_t st = (hipStream_t)stream;
 #define MM_LAUNCH_ROWS_PAIR(ACTV, CFG)                                                       \
   return launch_prefill2<false, ACTV, CFG, true>(a, K, Bg, sg, nullptr, Bu, su, nullptr,       \
                                                  (f16*)C, ldc, M, N, K, g, p.ksplit, part, st)

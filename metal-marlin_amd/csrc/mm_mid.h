@@ -85,11 +85,27 @@ MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
     const int p = min((i * NWAVE + wave) * 64 + lane, Sh::A_PIECES - 1);
     a_src[i] = src.arow(p / PPR) + 8 * ((p % PPR) ^ asw(p / PPR));
   }
+  // Marlin words: piece p is 4 columns of one word row, [16 word rows][BN].
+  // Row-packed words (ROWP): a column's 16 words of a chunk are 64 contiguous
+  // bytes, four pieces; piece pc of the q-th column in lane order lies at slot
+  // 4*q + (pc ^ ((q >> 2) & 3)), so a load instruction reads 64-byte runs and the
+  // lanes' LDS reads hit distinct banks.  Wave wk's two steps need piece wk
+  // only: lane half h takes its words 2h (step 0) and 2h + 1 (step 1), one 8-byte
+  // read per column, and the A pieces in the same k order.  4096 -> 2 x 14336 at
+  // M = 64 25.5 us, as the Marlin words (the prefill kernel took 35.2).
+  constexpr bool ROWP = is_rowpacked<Src>::value;
+  static_assert(!ROWP || (BK == 128 && WK == 4), "one piece of a column per wave");
   const uint32_t* b_src[Sh::B_IT];
 #pragma unroll
   for (int i = 0; i < Sh::B_IT; ++i) {
     const int p = min((i * NWAVE + wave) * 64 + lane, Sh::B_PIECES - 1);
-    b_src[i] = src.bcol(4 * (p % (BN / 4)), 4) + (size_t)(p / (BN / 4)) * ld;
+    if constexpr (ROWP) {
+      const int q = p >> 2, pc = (p & 3) ^ ((q >> 2) & 3);
+      const int P = TM ? q : (q & ~63) + 2 * (q & 31) + ((q >> 5) & 1);
+      b_src[i] = src.brow(P) + 4 * pc;
+    } else {
+      b_src[i] = src.bcol(4 * (p % (BN / 4)), 4) + (size_t)(p / (BN / 4)) * ld;
+    }
   }
   int s_row[Sh::S_IT];
   const f16* s_src[Sh::S_IT];
@@ -116,7 +132,7 @@ MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
 #pragma unroll
     for (int i = 0; i < Sh::B_IT; ++i) {
       const int wp = i * NWAVE + wave;
-      gl2lds16(b_src[i] + (size_t)(k0 / 8) * ld,
+      gl2lds16(b_src[i] + (ROWP ? (size_t)(k0 / 8) : (size_t)(k0 / 8) * ld),
                wp * 64 < Sh::B_PIECES ? base + Sh::B_OFF + wp * 1024 : smem + Sh::D_OFF);
     }
 #pragma unroll
@@ -144,13 +160,21 @@ MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
   f16x8 af[2][RB];
   f16x8 bq[2][CW];
   uint32_t wv[CW];
+  u32x2 wp[CW];              // ROWP: both steps' words
   f16 sc[CW] = {}, nz[CW] = {};
+  const uint32_t p_base = Sh::B_OFF + 64 * (wn * 64 + l32) + 16 * (wk ^ ((l32 >> 2) & 3)) + 8 * h;
   // LDS reads of step s (of this wave) of the chunk at ring position st.
   auto read = [&](int st, int s, int slot) {
     const int t = wk * STEPS + s;
     const char* const base = smem + st * Sh::STAGE;
     const uint32_t bo = b_base + t * 2 * BN * 4;
-    if constexpr (TM) {
+    if constexpr (ROWP) {
+#pragma unroll
+      for (int j = 0; j < CW; ++j) {
+        if (s == 0) wp[j] = *(const u32x2*)(base + p_base + j * 32 * 64);
+        wv[j] = wp[j][s];
+      }
+    } else if constexpr (TM) {
 #pragma unroll
       for (int j = 0; j < CW; ++j) wv[j] = *(const uint32_t*)(base + bo + j * CS * 4);
     } else {
@@ -160,7 +184,8 @@ MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
 #pragma unroll
     for (int rb = 0; rb < RBL; ++rb)
       af[slot][rb] =
-          *(const f16x8*)(base + a_base + rb * 32 * BK * 2 + (((2 * t + h) ^ asx) * 16));
+          *(const f16x8*)(base + a_base + rb * 32 * BK * 2 +
+                          (((ROWP ? 4 * wk + 2 * h + s : 2 * t + h) ^ asx) * 16));
   };
   auto read_scale = [&](int st, int k0) {
     // row of this wave's group among the staged rows

@@ -310,11 +310,24 @@ def test_mid_bit_exact(rng, M, K, N, g):
     # scales 8- but not 16-byte aligned: the prefill kernel's operands
     sv = torch.cat([td[2].reshape(-1)[:4], td[2].reshape(-1)])[4:].view(td[2].shape)
     _same(mmfp4.marlin_gemm_fp4(td[0], td[1], sv, g), ref)
+    rows = to_dev(np.ascontiguousarray(p.T))
+    if g % 64 == 0:
+        _same(mmfp4.mmfp4_gemm_rowpacked(td[0], rows, td[2], g), ref)
+        _same(mmfp4.mmfp4_gemm_rowpacked(td[0], rows, sv, g), ref)
     if N <= 1032:
         p2, s2 = _exact_fp4(rng, K, N, g)
         ref2 = ofp4.gemm_fp4_ref(a, p2, s2, g)
         out = mmfp4.fused_gate_up_gemm(*td, to_dev(p2), to_dev(s2), g)
         _same(out, np.concatenate([ref, ref2], 1))
+        if g % 64 == 0:
+            rows2, ds2, out = to_dev(np.ascontiguousarray(p2.T)), to_dev(s2), torch.empty_like(out)
+            ws = mmfp4._lib.workspace(
+                out.device, int(mmfp4._lib.load().mm_gemm_workspace_bytes(M, 2 * N, K)))
+            P = mmfp4._lib.ptr
+            mmfp4._lib.call("mm_fp4_gate_up_rowpacked", P(td[0]), P(rows), P(td[2]), P(rows2),
+                            P(ds2), P(out), M, N, K, g, 0, P(ws), ws.numel(),
+                            mmfp4._lib.stream_of(out))
+            _same(out, np.concatenate([ref, ref2], 1))
         n3 = max(8, N // 2 // 8 * 8)
         qkv = mmfp4.mmfp4_fused_qkv(*td, to_dev(p2), to_dev(s2),
                                     to_dev(p[:, :n3]), to_dev(s[:, :n3]), g)
