@@ -67,7 +67,8 @@ struct SkMulti {
 // fp32 with PW = N, 2N for the pair modes (gate at n, up at N + n), or ntot.
 // ROWP: 0 Marlin-layout weights; 1, 2 row-packed [N, K/8] weights with
 // scales [N, K/g] (1) or [K/g, N] (2), transposed through LDS into the
-// Marlin operand order (skinny_wave RT); 3 Marlin-layout weights with scales
+// Marlin operand order (skinny_wave RT) or, the pair with groups of 128 k or
+// more, read in place from LDS (skinny_wave_rows); 3 Marlin-layout weights with scales
 // [N, K/g].
 // Row-packed single-tile blocks: the RT staging takes a few registers over
 // the 128 that keep two 8-wave blocks resident per CU; at that limit the
@@ -144,7 +145,10 @@ k_skinny(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
                 : (t == 0 ? SkTile{B, S, Z, n0} : SkTile{B2, S2, Z2, n0});
   if constexpr (STAGE) {
     static_assert(!INT4 && ACT != SK_MULTI, "row-packed: FP4 product or gate/up pair");
-    skinny_wave<false, MT, NT, SPW, FL, false, ROWP == 1, false, true>(
+    if constexpr (!ONE && ROWP == 2 && MT == 1 && SPW == 8 && FL >= 4)
+      skinny_wave_rows<FL>(A, lda, M, tl, N, K, g, blk_st0 + wave * SPW, nrounds, NW * SPW, acc,
+                           (char*)red + wave * NT * 8192);
+    else skinny_wave<false, MT, NT, SPW, FL, false, ROWP == 1, false, true>(
         A, lda, nullptr, 1, M, tl, N, K, g, blk_st0 + wave * SPW, nrounds, NW * SPW, acc,
         nullptr, (char*)red + wave * NT * 8192);
     __syncthreads();   // every wave is done with its staging area
@@ -1492,8 +1496,8 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
   MM_CHECK_ARG(tiles <= SK_MAX_TILES, "%s: too many columns", who);
   if (M == 0) return 0;
   // Two-slab kernel where one product of the same width takes it (4096 ->
-  // 4096 + 1024 + 1024 at M = 1: 7.1 -> 6.1 us of the layer's call against the
-  // 64-column tiles and their split-K hand-off).
+  // 4096 + 1024 + 1024 at M = 1, against 64-column tiles: a layer's four calls
+  // 32.3 -> 31.3 us).
   if (use_dual(M, ntot, K, g))
     return launch_dual<false, false, true>(A, nullptr, nullptr, nullptr, nullptr, M, ntot, K, g,
                                            st, &mp);

@@ -27,6 +27,12 @@ namespace mmsk {
 
 constexpr int SK_COLS = 64;   // columns of one virtual-tile quad
 
+// 16 bytes per lane, global -> LDS at a wave-uniform base + 16 * lane, non-temporal.
+MM_DEV void gl2lds16_nt(const void* src, void* lds_base_uniform) {
+  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds_base_uniform,
+                                   16, 0, 2);
+}
+
 // Pre-scaled word decode (exact reference fp16 weights).
 template <bool INT4>
 struct WordDq;
@@ -395,6 +401,121 @@ MM_DEV void skinny_wave(const f16* __restrict__ A, int lda, const int* __restric
           }
       }
     }
+  }
+}
+
+// skinny_wave for the row-packed FP4 pair (two tiles, up to 16 rows, SPW == 8,
+// FL >= 4: groups of 128 k or more).  A round's words -- 8 16-byte pieces of 4
+// words per column -- go global -> LDS directly, with whole row segments, into
+// the wave's region `stage` (8 KiB per tile, the wave's own: no barrier), and a
+// lane reads its columns' words back a piece at a time.  Which words of a
+// 128-k block a lane takes is free as long as the activation operand follows,
+// so nothing is transposed: at steps 4*b .. 4*b + 3 lane group q takes the four
+// words of piece 4*b + q.  The next round is requested once this round's words
+// are in registers and travels during the math (staging through registers, the
+// RT form, has no room for that and spends 32 LDS stores per 8 loads).
+// Piece p of column 4c + j lies at 16-byte unit 8 * (16 * j + c) + (p ^ (c >> 1)):
+// the 16 lanes of an LDS read pass hit all banks.
+// Measured against RT, 4096 -> 2 x 14336, g = 128: M = 1 15.7 -> 14.1 us, M = 8
+// 16.0 -> 15.0, M = 16 16.4 both.  RT stays for the rest: with g = 64 the two are
+// equal (and this form spills registers at g = 32); single-tile products and
+// the pair at 17..32 rows are slower in this form (14336 -> 4096 M = 16 12.3 ->
+// 13.2, pair M = 32 22.7 -> 25.4: an activation load touches four lines per row
+// where RT's order touches one).
+template <int FL>
+MM_DEV void skinny_wave_rows(const f16* __restrict__ A, int lda, int M, const SkTile (&tl)[2],
+                             int N, int K, int g, int st0, int nrounds, int ststride,
+                             f32x4 (&acc)[1][2][4], char* stage) {
+  constexpr int SPW = 8, NT = 2, NF = SPW / FL;
+  static_assert(FL == 4 || FL == 8, "whole 128-k blocks per group");
+  const int lane = threadIdx.x & 63;
+  const int c = lane & 15, q = lane >> 4;
+  const int KP = K >> 3, nsteps = (KP + 3) / 4;
+  auto word_row = [&](int i) { return 16 * (i / 4) + 4 * q + i % 4; };   // of a round
+  const __amdgpu_buffer_rsrc_t ars = mm_rsrc(A);   // rows past M: see skinny_wave
+  const uint32_t aoff = c < M ? (uint32_t)c * (uint32_t)lda * 2u : MM_DEAD_OFFSET;
+  const uint32_t coff = (uint32_t)min(tl[0].col0 + 4 * c, N - 4);   // both tiles
+  st0 = __builtin_amdgcn_readfirstlane(st0);
+  f16x8 a[SPW];
+  f16x4 s4[NF][NT];
+  u32x4 w[SPW][NT];
+  // Steps past K multiply the column's last words by zero activations.
+  auto load_operands = [&](int stb) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const uint32_t gi = (uint32_t)((min(stb + f * FL, nsteps - 1) * 32) / g);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) s4[f][t] = load_scales4<false>(tl[t].S, gi, coff, N, K / g);
+    }
+#pragma unroll
+    for (int i = 0; i < SPW; ++i) {
+      const int kp = 4 * stb + word_row(i);
+      a[i] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                                           ars, kp < KP ? aoff + (uint32_t)kp * 16u : MM_DEAD_OFFSET,
+                                           0, 0));
+    }
+  };
+  auto issue_words = [&](int stb) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < SPW; ++i) {
+        const int u = 64 * i + lane, s = u / 8;
+        const int p = (u & 7) ^ ((s >> 1) & 7);
+        const uint32_t cg = (uint32_t)min(tl[t].col0 + 4 * (s & 15) + (s >> 4), N - 1);
+        const uint32_t kw = (uint32_t)min(4 * stb + 4 * p, KP - 4);
+        gl2lds16_nt(at_bytes<uint32_t>(tl[t].B, (cg * (uint32_t)KP + kw) * 4u),
+                    stage + 8192 * t + 1024 * i);
+      }
+  };
+  if (st0 >= nsteps) return;
+  issue_words(st0);
+  load_operands(st0);
+  for (int r = 0; r < nrounds; ++r) {
+    const int stb = st0 + r * ststride;    // wave-uniform
+    if (stb >= nsteps) break;
+    const bool more = r + 1 < nrounds && stb + ststride < nsteps;
+    __builtin_amdgcn_s_waitcnt(0xF70);     // vmcnt(0): this round has arrived
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int b = 0; b < SPW / 4; ++b) {
+          const u32x4 x = *(const u32x4*)(stage + 8192 * t +
+                                          16 * (8 * (16 * j + c) + ((4 * b + q) ^ (c >> 1))));
+#pragma unroll
+          for (int k = 0; k < 4; ++k) w[4 * b + k][t][j] = x[k];
+        }
+    if (more) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the words are in registers
+      asm volatile("" ::: "memory");
+      issue_words(stb + ststride);
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      f32x4 grp[NT][4];
+#pragma unroll
+      for (int i = f * FL; i < (f + 1) * FL; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            grp[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                a[i], raw_fp4_word(w[i][t][j]), i == f * FL ? f32x4{0, 0, 0, 0} : grp[t][j], 0, 0,
+                0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[0][t][j] += (float)sanitize_scale(s4[f][t][j]) * grp[t][j];
+    }
+    // The next round's activations and scales come from the caches: requested
+    // after the math they arrive before its words do, and need no second set
+    // of registers.
+    if (more) load_operands(stb + ststride);
   }
 }
 

@@ -364,3 +364,26 @@ def test_multi_qkv_two_slab(rng, M, K, Ns):
     out = mmfp4.mmfp4_fused_qkv(a, *[to_dev(t) for pair in w for t in pair], g)
     for o, (p, s) in zip(out, w):
         _same(o, ofp4.gemm_fp4_ref(to_np(a), p, s, g))
+
+
+@pytest.mark.parametrize("M,K,N,g", [
+    (1, 128, 8, 128), (2, 384, 72, 128), (7, 4096, 1032, 128), (16, 2176, 200, 128),
+    (15, 2560, 136, 256), (9, 1024, 6408, 512), (3, 14336, 64, 1024),
+])
+def test_rowpacked_pair_decode(rng, M, K, N, g):
+    """Row-packed pair at decode sizes, groups of 128 and more: rounds that
+    overhang K, columns that end inside a tile, one and several rounds per wave,
+    with and without a K split."""
+    import mmfp4
+    w = [_exact_fp4(rng, K, N, g) for _ in range(2)]
+    a = _acts(rng, M, K)
+    ref = np.concatenate([ofp4.gemm_fp4_ref(a, p, s, g) for p, s in w], 1)
+    announce(f"exact row-packed pair M={M} K={K} N={N} g={g}")
+    da = to_dev(a)
+    ops = [to_dev(t) for p, s in w for t in (np.ascontiguousarray(p.T), s)]
+    out = torch.empty((M, 2 * N), dtype=torch.float16, device="cuda")
+    lib = mmfp4._lib
+    ws = lib.workspace(out.device, int(lib.load().mm_gemm_workspace_bytes(M, 2 * N, K)))
+    lib.call("mm_fp4_gate_up_rowpacked", lib.ptr(da), *map(lib.ptr, ops), lib.ptr(out), M, N, K, g,
+             0, lib.ptr(ws), ws.numel(), lib.stream_of(da))
+    _same(out, ref)
