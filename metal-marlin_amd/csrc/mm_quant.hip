@@ -291,14 +291,16 @@ k_u4_quantize(const f16* __restrict__ Wt, int N, int K, int g,
 // x / a, correctly rounded, for r = RN(1 / a): one Newton step on the quotient
 // with an exact remainder (Markstein, "Computation of elementary functions on
 // the IBM RISC System/6000 processor", 1990).  Its conditions -- no overflow or
-// underflow on the way -- hold for a in [1e-7, 2^100] (both quantizers floor
+// underflow on the way -- hold for a in [1e-7, 2^40] (both quantizers floor
 // their divisor at 1e-7) and |x| that is zero or at least 2^-80; for fp16 x the
-// latter always holds.
+// latter always holds.  A quotient is then zero or at least 2^-120 and a
+// remainder at least 2^-126, both normal; a negative x never gives -0, which
+// fp4_ties_down must not get.
 MM_DEV float div_by(float x, float a, float r) {
   const float q = x * r;
   return __builtin_fmaf(__builtin_fmaf(-q, a, x), r, q);
 }
-MM_DEV bool div_ok(float a) { return a <= 0x1p100f; }
+MM_DEV bool div_ok(float a) { return a <= 0x1p40f; }
 
 // Moves v one step toward zero and sets its last bit: the hardware's
 // round-to-even FP4 convert then sends a midpoint down, as e2m1_nearest does,

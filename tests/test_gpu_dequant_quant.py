@@ -231,3 +231,23 @@ def test_dequant_widths(rng, N):
     assert np.array_equal(out.view(np.uint16), ofp4.dequant_fp4(packed, s, g).view(np.uint16))
     out = to_np(mmfp4.dequant_int4(to_dev(packed), to_dev(s), to_dev(z), K, N, g))
     assert np.array_equal(out.view(np.uint16), ofp4.dequant_u4(packed, s, z, g).view(np.uint16))
+
+
+@pytest.mark.parametrize("e", [38, 39, 40, 41, 69, 70, 71, 90, 100, 101, 126])
+def test_quantize_fp4_wide_float32_groups(rng, e):
+    """float32 groups whose largest weight is 2^e beside small ones of both signs,
+    down to and past 2^-80: around the divisor limit of the tiled quantizer, and
+    where the quotient underflows to -0 (code 0)."""
+    import mmfp4
+    N, K, g = 64, 1024, 128
+    w = np.ldexp(rng.uniform(1, 2, (N, K)), rng.integers(-82, min(e, 40), (N, K))).astype(np.float32)
+    w[:, ::3] = np.ldexp(1.0, -80)
+    w[:, 1::16] = np.ldexp(1.0, -60)
+    w *= rng.choice([-1, 1], (N, K)).astype(np.float32)
+    w[:, ::g] = np.ldexp(1.0, e)
+    announce(f"quantize float32 absmax 2^{e}")
+    with np.errstate(all="ignore"):
+        rp, rs = ofp4.quantize_fp4(w, g)
+    packed, s = mmfp4.quantize_fp4(to_dev(w), group_size=g)
+    assert np.array_equal(to_np(s).view(np.uint16), rs.view(np.uint16))
+    assert np.array_equal(to_np(packed).view(np.uint32), rp)
