@@ -479,9 +479,9 @@ k_moe_grouped(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
 // ---------------------------------------------------------------------------
 // Grouped expert GEMM, prefill-sized groups: the pipelined MFMA main loop of
 // the dense prefill kernel (mm_prefill.h) over one (expert, row tile,
-// column tile) per block.  grid.y enumerates row tiles of BM rows over all
-// experts in expert order; each block finds its expert with one wave scan of
-// the offsets (grid.y is an upper bound; surplus blocks exit).  A rows are
+// column tile) per block.  The grid is an upper bound of these pairs; each block
+// finds its own from the experts' row counts (wave scans of the offsets), the
+// fullest row tiles first, and surplus blocks exit.  A rows are
 // gathered through sorted_idx (gather=1) or read in sorted order.  Column
 // map (tile-major, CW=2): each wave's 64 LDS columns are 32 output columns
 // twice -- act=1: the gate columns then the matching up columns (N/2 on),
@@ -516,7 +516,7 @@ template <int WM, int WN, int RB, bool G64, int STAGES>
 __global__ void __launch_bounds__(WM * WN * 64, MOE_PF_WAVES_PER_SIMD)
 k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
               const int32_t* __restrict__ offsets, int gather, int topk, ExpertW W, int E,
-              int K, int N, int g, int act, int gx, int run, f16* __restrict__ Y) {
+              int K, int N, int g, int act, int gx, f16* __restrict__ Y) {
   constexpr int CW = 2;
   constexpr int SROWS = G64 ? PF2_SROWS_G64 : PF2_SROWS;
   using Sh = Pf2Shape<false, WM, WN, RB, CW, STAGES, SROWS>;
@@ -563,15 +563,30 @@ k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
     if (lane == 0) t[0] = 0;
   }
   __syncthreads();
-  // Blocks are dealt round-robin to the 8 XCDs: XCD x takes every eighth run of
-  // `run` row tiles (the tiles an expert has on average, which share its weights
-  // in that XCD's L2), each tile with its gx column tiles, which share its A
-  // rows.  The grid is an upper bound; blocks past the last tile exit.
-  const int L = blockIdx.x;
-  const int yx = (L >> 3) / gx, bx = (L >> 3) - yx * gx;
-  int y = (yx / run * 8 + (L & 7)) * run + yx % run;
-  int c = RB - 1;
-  while (c >= 0 && y >= tp[c * (E + 1) + E]) y -= tp[c * (E + 1) + E], --c;
+  // Blocks are dealt round-robin to the 8 XCDs (L & 7).  Every XCD takes an equal,
+  // contiguous share of each class's (row tile, column tile) pairs, largest class
+  // first: the column tiles of a row tile share its A rows, and neighbouring row
+  // tiles their expert's weights, in that XCD's L2.  A class's share is uneven by
+  // one pair at most; where the surplus of one class ends the next one's starts.
+  // The grid is an upper bound; blocks past the last pair exit.  Dealing whole
+  // runs of an expert's average tile count in place of equal shares left XCDs
+  // idle when there were few experts (one expert on one XCD).  Whole MLP, runs
+  // against shares (in brackets: shares in plain expert order): 1 expert, T = 2048
+  // 160 -> 62 us (64); 4 experts, T = 2048 181 -> 109 (119); 16 experts 123 -> 115
+  // (119); 128 experts, T = 1024 152 -> 148 (167).
+  int p = (int)blockIdx.x >> 3, y = 0, bx = 0, c = RB - 1, first = 0;
+  for (; c >= 0; --c) {
+    const int n = tp[c * (E + 1) + E] * gx, q = n >> 3, rem = n & 7;
+    const int x = ((int)(blockIdx.x & 7) - first) & 7;
+    if (p < q + (x < rem)) {
+      const int lin = x * q + min(x, rem) + p;
+      y = lin / gx;
+      bx = lin - y * gx;
+      break;
+    }
+    p -= q + (x < rem);
+    first += rem;
+  }
   if (c < 0) return;
   const int* const tc = tp + c * (E + 1);
   int lo = 0, hi = E - 1;            // expert e with tc[e] <= y < tc[e + 1]
@@ -579,10 +594,16 @@ k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
     const int mid = (lo + hi + 1) >> 1;
     if (tc[mid] <= y) lo = mid; else hi = mid - 1;
   }
-  const int e = lo;
-  const int r0 = offsets[e], r1 = offsets[e + 1];
+  // All uniform.  Declared so, here and in the main loop (UW): it has no vector
+  // register to spare, and a spill inside it waits for the loads in flight (one to
+  // three reloads there: 1 expert, T = 96 58-64 us, none 54.5).
+  const int e = __builtin_amdgcn_readfirstlane(lo);
+  bx = __builtin_amdgcn_readfirstlane(bx);
+  const int r0 = __builtin_amdgcn_readfirstlane(offsets[e]);
+  const int r1 = __builtin_amdgcn_readfirstlane(offsets[e + 1]);
   // Full tiles come first in an expert; only class RB - 1 holds more than one.
-  const int mb = r0 + (c == RB - 1 ? y - tc[e] : (r1 - r0) / BM) * BM;
+  const int mb =
+      __builtin_amdgcn_readfirstlane(r0 + (c == RB - 1 ? y - tc[e] : (r1 - r0) / BM) * BM);
   __syncthreads();                   // the prefixes have been read: the ring may start
   const int rows = min(BM, r1 - mb);
   const int half = N / 2;
@@ -598,8 +619,8 @@ k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
       [&](auto lc) {
         constexpr int L = decltype(lc)::value;
         if (rb_live == L)
-          pf2_mainloop<false, WM, WN, RB, CW, G64, true, STAGES, SROWS, L>(src, K, g, 0,
-                                                                           K / PF2_BK, smem, acc);
+          pf2_mainloop<false, WM, WN, RB, CW, G64, true, STAGES, SROWS, L, true>(
+              src, K, g, 0, K / PF2_BK, smem, acc);
       },
       std::make_integer_sequence<int, RB + 1>{});
 
@@ -764,18 +785,17 @@ int grouped_gemm(const uint16_t* X, const int32_t* sorted_idx, const int32_t* of
   do {                                                                                         \
     constexpr int BM = WM * 32 * RB, BN = WN * 64;                                             \
     const int gx = act ? mm_cdiv(nout, BN / 2) : mm_cdiv(N, BN);                               \
-    const long run = std::max<long>(1, tk / ((long)E * BM));                                   \
     const long tiles = (tk + BM - 1) / BM + std::min<long>(E, tk);                             \
-    const long blocks = (long)gx * ((tiles + 8 * run - 1) / (8 * run) * (8 * run));            \
+    const long blocks = ((long)gx * tiles + 7) / 8 * 8;                                        \
     MM_CHECK_ARG(blocks < (1L << 30), "mm_moe_grouped_gemm: T*k=%ld too large", tk);           \
     if (g % PF2_BK == 0)                                                                       \
       hipLaunchKernelGGL((k_moe_prefill<WM, WN, RB, true, ST>), dim3((unsigned)blocks), \
                          dim3(WM * WN * 64), 0, (hipStream_t)stream, (const f16*)X, sorted_idx, \
-                         offsets, gather, k, W, E, K, N, g, act, gx, (int)run, (f16*)Y);  \
+                         offsets, gather, k, W, E, K, N, g, act, gx, (f16*)Y);            \
     else                                                                                       \
       hipLaunchKernelGGL((k_moe_prefill<WM, WN, RB, false, ST>), dim3((unsigned)blocks),\
                          dim3(WM * WN * 64), 0, (hipStream_t)stream, (const f16*)X, sorted_idx, \
-                         offsets, gather, k, W, E, K, N, g, act, gx, (int)run, (f16*)Y);  \
+                         offsets, gather, k, W, E, K, N, g, act, gx, (f16*)Y);            \
   } while (0)
     if (cfg == 1)
       MM_LAUNCH_MOE_PF(1, 4, 2, MOE_PF_STAGES);    // 64 x 256, 4 waves

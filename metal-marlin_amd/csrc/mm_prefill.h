@@ -110,9 +110,14 @@ struct Pf2Shape {
 // branch splits the MFMA stream from the interleaved LDS reads and decode;
 // callers with a per-wave count switch over it once, outside the loop.  The
 // wave still issues its share of the loads and joins every barrier.
+// UW: the wave number is declared uniform, so the LDS addresses that the loads go
+// to stay in scalar registers (about 8 vector registers fewer; the grouped kernel
+// spills in its loop otherwise).  The dense tiles, which do not spill, measured
+// both better and worse with it (M = 2048 layer 820 -> 811 us, M = 8192 row-packed
+// MLP 2438 -> 2470) and keep it off.
 // Requires K % 64 == 0.
 template <bool INT4, int WM, int WN, int RB, int CW, bool G64, bool TM, int STAGES, int SROWS,
-          int RBL = RB, class Src>
+          int RBL = RB, bool UW = false, class Src>
 MM_DEV void pf2_mainloop(const Src& src, int K, int g, int c_beg, int c_end, char* smem,
                          f32x16 (&acc)[RB][CW]) {
   static_assert(RBL >= 0 && RBL <= RB, "live row blocks");
@@ -122,7 +127,8 @@ MM_DEV void pf2_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
   constexpr int A_IT = Sh::A_IT, B_IT = Sh::B_IT, S_IT = Sh::S_IT;
   constexpr int A_BYTES = Sh::A_BYTES, B_BYTES = Sh::B_BYTES, S_BYTES = Sh::S_BYTES;
   constexpr int B_OFF = Sh::B_OFF, S_OFF = Sh::S_OFF, Z_OFF = Sh::Z_OFF, D_OFF = Sh::D_OFF;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = UW ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
   const int l32 = lane & 31, h = lane >> 5;
   const int nch = c_end;
