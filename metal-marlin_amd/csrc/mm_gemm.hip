@@ -281,13 +281,11 @@ k_skinny(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
 // grid of narrow layers without a K split.
 // ROWP: row-packed FP4 words [N, K/8] (K % 512 == 0), transposed through
 // LDS into the Marlin operand order (skinny_wave RT); scales [N, K/g] when
-// SROW, else [K/g, N].  MULTI: the tiles of up to three matrices in turn (mp).
-template <int INT4, int SPW, int NW, int FL, bool SROW = false, bool ROWP = false,
-          bool MULTI = false>
-__global__ void __launch_bounds__(NW * 64)
-k_skinny_dual(const f16* __restrict__ A, const uint32_t* __restrict__ B,
-              const f16* __restrict__ S, const f16* __restrict__ Z, f16* __restrict__ C, int M,
-              int N, int K, int g, int nrounds, SkMulti mp) {
+// SROW, else [K/g, N].
+template <int INT4, int SPW, int NW, int FL, bool SROW, bool ROWP>
+MM_DEV void skinny_dual(const f16* __restrict__ A, const uint32_t* __restrict__ B,
+                        const f16* __restrict__ S, const f16* __restrict__ Z,
+                        f16* __restrict__ C, int M, int N, int K, int g, int nrounds, int tile) {
   // ROWP: each wave stages its weights through 8 KiB of LDS in the main
   // loop; the block reduction reuses the same memory afterwards.
   constexpr int RED = row_items_lds_floats<1, 1, NW>();
@@ -295,15 +293,6 @@ k_skinny_dual(const f16* __restrict__ A, const uint32_t* __restrict__ B,
   __shared__ __attribute__((aligned(16))) float red[LDSF];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, q = lane >> 4;
-  int tile = blockIdx.x;
-  if constexpr (MULTI) {
-    const int p = tile >= mp.tile0[2] ? 2 : (tile >= mp.tile0[1] ? 1 : 0);
-    B = mp.B[p];
-    S = mp.S[p];
-    C = mp.C[p];
-    N = mp.N[p];
-    tile -= mp.tile0[p];
-  }
   const int n0 = tile * 32;
   f32x4 acc[1][1][4];
 #pragma unroll
@@ -334,6 +323,26 @@ k_skinny_dual(const f16* __restrict__ A, const uint32_t* __restrict__ B,
     if (q < 2 && c < 8 && row < M && col < N)
       *(f16x4*)(C + (size_t)row * N + col) = f16x4{(f16)v[0], (f16)v[1], (f16)v[2], (f16)v[3]};
   }
+}
+
+template <int INT4, int SPW, int NW, int FL, bool SROW = false, bool ROWP = false>
+__global__ void __launch_bounds__(NW * 64)
+k_skinny_dual(const f16* __restrict__ A, const uint32_t* __restrict__ B,
+              const f16* __restrict__ S, const f16* __restrict__ Z, f16* __restrict__ C, int M,
+              int N, int K, int g, int nrounds) {
+  skinny_dual<INT4, SPW, NW, FL, SROW, ROWP>(A, B, S, Z, C, M, N, K, g, nrounds, blockIdx.x);
+}
+
+// The tiles of up to three FP4 matrices in turn.  A kernel of its own: the table is
+// 144 bytes of launch arguments, which the smallest product (4096 x 4096, M = 1)
+// paid for without reading them: enqueueing it took 5.04 us against 4.88.
+template <int SPW, int NW, int FL>
+__global__ void __launch_bounds__(NW * 64)
+k_skinny_dual_multi(const f16* __restrict__ A, int M, int K, int g, int nrounds, SkMulti mp) {
+  const int t = blockIdx.x;
+  const int p = t >= mp.tile0[2] ? 2 : (t >= mp.tile0[1] ? 1 : 0);
+  skinny_dual<0, SPW, NW, FL, false, false>(A, mp.B[p], mp.S[p], nullptr, mp.C[p], M, mp.N[p], K,
+                                            g, nrounds, t - mp.tile0[p]);
 }
 
 // Column-strip kernel (M <= 16, group size a multiple of 32): one block per
@@ -1009,25 +1018,16 @@ bool use_dual(int M, int N, int K, int g) {
          mm_cdiv(N, SK_COLS) < MM_SK_DUAL_BELOW && mm_cdiv(N, 32) >= MM_SK_DUAL_MIN_TILES;
 }
 
-template <int INT4, bool SROW = false, bool MULTI = false>
+template <int INT4, bool SROW = false>
 int launch_dual(const f16* A, const uint32_t* B, const f16* S, const f16* Z, f16* C, int M, int N,
-                int K, int g, hipStream_t st, SkMulti* mp = nullptr) {
+                int K, int g, hipStream_t st) {
   constexpr int SPW = MM_SK_DUAL_SPW, NW = MM_SK_DUAL_NW;
   const int nsteps = K / 64;                           // 64-k steps
   const int nrounds = mm_cdiv(nsteps, NW * SPW);
   const int fl = flush_steps(g / 2, SPW);              // 64-k steps per scale group
-  int tiles = mm_cdiv(N, 32);
-  if (MULTI) {
-    tiles = 0;
-    for (int i = 0; i < 3; ++i) {
-      mp->tile0[i] = tiles;
-      tiles += mm_cdiv(mp->N[i], 32);
-    }
-  }
-  const SkMulti none{};
 #define MM_LAUNCH_DU(FLV)                                                                      \
-  hipLaunchKernelGGL((k_skinny_dual<INT4, SPW, NW, FLV, SROW, false, MULTI>), dim3(tiles),       \
-                     dim3(NW * 64), 0, st, A, B, S, Z, C, M, N, K, g, nrounds, MULTI ? *mp : none)
+  hipLaunchKernelGGL((k_skinny_dual<INT4, SPW, NW, FLV, SROW>), dim3(mm_cdiv(N, 32)), dim3(NW * 64), 0, \
+                     st, A, B, S, Z, C, M, N, K, g, nrounds)
   switch (fl) {
     case 1: MM_LAUNCH_DU(1); break;
     case 2: MM_LAUNCH_DU(2); break;
@@ -1037,6 +1037,30 @@ int launch_dual(const f16* A, const uint32_t* B, const f16* S, const f16* Z, f16
   }
 #undef MM_LAUNCH_DU
   MM_CHECK_LAUNCH("gemm(dual)");
+  return 0;
+}
+
+// The same over mp's matrices.
+int launch_dual_multi(const f16* A, int M, int K, int g, hipStream_t st, SkMulti* mp) {
+  constexpr int SPW = MM_SK_DUAL_SPW, NW = MM_SK_DUAL_NW;
+  const int nrounds = mm_cdiv(K / 64, NW * SPW);
+  int tiles = 0;
+  for (int i = 0; i < 3; ++i) {
+    mp->tile0[i] = tiles;
+    tiles += mm_cdiv(mp->N[i], 32);
+  }
+#define MM_LAUNCH_DUM(FLV)                                                                     \
+  hipLaunchKernelGGL((k_skinny_dual_multi<SPW, NW, FLV>), dim3(tiles), dim3(NW * 64), 0, st, A, M, K, \
+                     g, nrounds, *mp)
+  switch (flush_steps(g / 2, SPW)) {
+    case 1: MM_LAUNCH_DUM(1); break;
+    case 2: MM_LAUNCH_DUM(2); break;
+    case 4: MM_LAUNCH_DUM(4); break;
+    case 8: MM_LAUNCH_DUM(8 <= SPW ? 8 : 4); break;
+    default: MM_CHECK_ARG(false, "gemm(dual): unsupported group size %d", g);
+  }
+#undef MM_LAUNCH_DUM
+  MM_CHECK_LAUNCH("gemm(dual, multi)");
   return 0;
 }
 
@@ -1499,8 +1523,7 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
   // 4096 + 1024 + 1024 at M = 1, against 64-column tiles: a layer's four calls
   // 32.3 -> 31.3 us).
   if (use_dual(M, ntot, K, g))
-    return launch_dual<false, false, true>(A, nullptr, nullptr, nullptr, nullptr, M, ntot, K, g,
-                                           st, &mp);
+    return launch_dual_multi(A, M, K, g, st, &mp);
   if (M > 16)
     return launch_skinny<false, 2, SK_MULTI>(A, K, nullptr, nullptr, nullptr, nullptr, nullptr,
                                              nullptr, nullptr, 0, M, ntot, K, g, ws, ws_bytes, st,
@@ -1611,7 +1634,7 @@ extern "C" int mm_fp4_gemm_rowpacked(const uint16_t* A, const uint32_t* B, const
 #define MM_LAUNCH_RDU(FLV, SR)                                                                  \
   hipLaunchKernelGGL((k_skinny_dual<false, 8, NW, FLV, SR, true>), dim3(mm_cdiv(N, 32)),       \
                      dim3(NW * 64), 0, st, (const f16*)A, B, (const f16*)S, nullptr, (f16*)C, M,  \
-                     N, K, g, nr, SkMulti{})
+                     N, K, g, nr)
 #define MM_LAUNCH_RDU_FL(SR)                                                                    \
   switch (fl) {                                                                                \
     case 1: MM_LAUNCH_RDU(1, SR); break;                                                       \
