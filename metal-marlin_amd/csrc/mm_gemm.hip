@@ -25,6 +25,7 @@
 #include "mm_skinny.h"
 #include "mm_prefill.h"
 #include "mm_mid.h"
+#include "mm_plan.h"
 
 // ===========================================================================
 // Skinny path
@@ -32,6 +33,9 @@
 namespace {
 using namespace mmsk;
 using namespace mmpf;
+using namespace mmplan;
+
+static_assert(PLAN_PF_BK == PF2_BK && PLAN_MID_BK == mmmid::MID_BK, "chunks of the plans");
 
 constexpr int SK_RED_BATCH = 8;   // partial-sum loads in flight per thread
 
@@ -1114,95 +1118,6 @@ int launch_prefill(const f16* A, int lda, const uint32_t* B, const f16* S, const
 #define PF2_MID 2, 4, 2, 2       // 128 x 256, 8 waves of 64 x 64
 #define PF2_SMALL 1, 4, 2, 2     // 64 x 256, 4 waves of 64 x 64
 
-#ifndef MM_PF_KS_BLOCKS
-#define MM_PF_KS_BLOCKS 200   // split K while the grid has fewer blocks than this
-#endif
-// Time of a grid of `blocks` 256-column prefill tiles of `rows` (256 or 128)
-// rows, in us at K = 4096 (it scales with K): one tile per CU, so whole rounds
-// of 256 and a last one that is little cheaper when it is not full.  Fitted to
-// FP4 measurements under sustained load (the clock is power limited):
-//   256 x 256: 96 blocks 98, 192 116, 288 210, 448 241, 512 263, 896 470, 3584 1710
-//   128 x 256: 128 blocks 61, 192 66, 256 73, 264 120, 384 135, 512 152, 1792 508
-double prefill_us(long blocks, int rows) {
-  const long full = blocks / 256, rem = blocks % 256;
-  if (rows == 256) return 3 + 117.0 * full + (rem ? 88 + 0.115 * rem : 0);
-  return 3 + 70.0 * full + (rem ? 54 + 0.07 * rem : 0);
-}
-
-// Prefill plan: tile config (0: 256x256, 1: 128x256, 2: 64x256) and K split.
-struct PrefillPlan {
-  int cfg;
-  int ksplit;
-  double us;   // at K = 4096, unsplit
-};
-
-PrefillPlan plan_prefill(int M, int N, int K) {
-  PrefillPlan p;
-  static const int BMs[3] = {256, 128, 64};
-  const long ct = mm_cdiv(N, 256);
-  const double big = prefill_us(mm_cdiv(M, 256) * ct, 256);
-  p.us = prefill_us(mm_cdiv(M, 128) * ct, 128);
-  p.cfg = M > 64 ? 1 : 2;
-  if (M > 128 && big < p.us) p.cfg = 0, p.us = big;
-  const long blocks = (long)mm_cdiv(M, BMs[p.cfg]) * ct;
-  // Split K when the grid cannot fill the 256 CUs; every split keeps >= 8
-  // chunks of 64 k so the pipeline stays full.  (256 x 256 tiles are taken only
-  // where one round of them beats two of 128 x 256.)
-  const int nch = K / PF2_BK;
-  int ks = 1;
-  if (p.cfg != 0)
-    while (blocks * ks < MM_PF_KS_BLOCKS && nch / (ks * 2) >= 8) ks *= 2;
-  p.ksplit = ks;
-  return p;
-}
-
-size_t prefill_ws_bytes(int M, int N, int K) {
-  const PrefillPlan p = plan_prefill(M, N, K);
-  return p.ksplit > 1 ? (size_t)p.ksplit * M * N * sizeof(float) : 0;
-}
-
-// Mid plan.  Tiles of 64 rows x 128 columns (8 waves, two blocks per CU), K split
-// while that fits one block per CU and leaves each split 8 chunks; 64 columns
-// where the split grid still leaves half the CUs idle; 128 rows where 65..128
-// rows have more 64-row tiles than CUs.  Measured on MI355X, FP4 g = 128, us
-// before (prefill tiles) -> mid:
-//   M = 64:  4096 -> 2 x 14336 (SwiGLU) 31.5 -> 24.3, 4096 -> 6144 18.8 -> 12.1,
-//            4096 -> 4096 17.0 -> 10.7, 4096 -> 1024 13.9 -> 9.4
-//   M = 100: 4096 -> 2 x 14336 43.1 -> 35.6, 4096 -> 4096 20.9 -> 13.1,
-//            14336 -> 4096 28.0 -> 24.1
-//   M = 512: 4096 -> 4096 31.8 -> 22.1; INT4 4096 -> 6144 59.6 -> 50.5
-//   row-packed M = 100: 4096 -> 2 x 14336 44.2 -> 35.2, 14336 -> 4096 28.0 -> 22.3;
-//            M = 300 122.8 -> 93.6 and 67.4 -> 52.8
-// What bounds it is LDS traffic and the matrix cores together.  Its time grows
-// smoothly with the tile count, the prefill tiles' in rounds of 256, so above
-// 128 rows the two are compared (mid_us, prefill_us): M = 512, 4096 -> 6144
-// 48.4 -> 35.7 mid, but M = 2048, 4096 -> 4096 prefill 73 against 81.
-struct MidPlan {
-  int rb, wn;   // 32-row blocks and 64-column groups per tile; wn == 0: not a mid-sized product
-  int ks, cps;  // K splits, chunks per split
-};
-
-// Time of `tiles` 64 x 128 tiles, as prefill_us: 512 tiles 44.6 us, 896 76, 1152 96,
-// 1536 120, 2256 177.
-double mid_us(long tiles) { return 4 + tiles * (20.0 / 256); }
-
-// ct: 128-column tiles of the product (the pair and multi forms count their own).
-MidPlan plan_mid_tiles(int M, long ct, int K) {
-  MidPlan p{2, 0, 1, 0};
-  const int nch = K / mmmid::MID_BK;
-  const long tiles = ct * mm_cdiv(M, 64);
-  if (M <= 32 || K % mmmid::MID_BK != 0 || nch < 4) return p;
-  if (M > 128 && tiles > 256 && mid_us(tiles) > plan_prefill(M, ct * 128, K).us) return p;
-  p.wn = 2;
-  if (M > 64 && M <= 128 && tiles > 256) p.rb = 4;
-  while (tiles * (p.ks + 1) <= 256 && nch / (p.ks + 1) >= 8) ++p.ks;
-  p.cps = mm_cdiv(nch, p.ks);
-  p.ks = mm_cdiv(nch, p.cps);
-  if (tiles * p.ks <= 128) p.wn = 1;
-  return p;
-}
-MidPlan plan_mid(int M, int N, int K) { return plan_mid_tiles(M, mm_cdiv(N, 128), K); }
-
 // Workspace of the plans that a product of these sizes can take: plain over N
 // columns, the pair over 2 x (N / 2), or two or three matrices of N columns in
 // all (up to two more partial tiles).
@@ -1365,13 +1280,13 @@ int gemm_dispatch(const char* who, const f16* A, const uint32_t* B, const f16* S
   if (off32 && M <= 32)
     return launch_skinny<INT4, 2, SK_PLAIN>(A, K, B, Sd, Z, nullptr, nullptr, nullptr, C, N, M, N,
                                             K, g, ws, ws_bytes, st);
-  if (const MidPlan mid = plan_mid(M, N, K); mid.wn != 0 && mid_ok<U4>(S, Z, N, g))
+  if (const MidPlan mid = plan_mid(M, N, K, g, U4); mid.wn != 0 && mid_ok<U4>(S, Z, N, g))
     return launch_mid<U4, SK_PLAIN>(mid, A, B, S, Z, nullptr, nullptr, nullptr, C, N, M, N, K, g,
                                     ws, ws_bytes, st);
   // The pipelined kernel stages scale rows in 8-column pieces (N % 8 == 0)
   // and whole 64-k chunks (K % 64 == 0).
   if (N % 8 == 0 && K % PF2_BK == 0) {
-    const PrefillPlan p = plan_prefill(M, N, K);
+    const PrefillPlan p = plan_prefill(M, N, K, g, U4);
     float* part = nullptr;
     if (p.ksplit > 1) {
       const size_t need = SK_COUNTER_BYTES + prefill_ws_bytes(M, N, K);
@@ -1432,11 +1347,11 @@ int pair_dispatch(const char* who, const f16* A, const uint32_t* Bg, const f16* 
   if (off32 && M <= 32)
     return launch_skinny<INT4, 2, ACT>(A, K, Bg, Sg, Zg, Bu, Su, Zu, C, ldc, M, N, K, g, ws,
                                        ws_bytes, st);
-  if (const MidPlan mid = plan_mid(M, 2 * N, K);
+  if (const MidPlan mid = plan_mid(M, 2 * N, K, g, INT4);
       mid.wn != 0 && mid_ok<INT4>(Sg, Zg, N, g) && mid_ok<INT4>(Su, Zu, N, g))
     return launch_mid<INT4, ACT>(mid, A, Bg, Sg, Zg, Bu, Su, Zu, C, ldc, M, N, K, g, ws, ws_bytes,
                                  st);
-  const PrefillPlan p = plan_prefill(M, 2 * N, K);
+  const PrefillPlan p = plan_prefill(M, 2 * N, K, g, INT4);
   float* part = nullptr;
   if (p.ksplit > 1) {
     const size_t need = SK_COUNTER_BYTES + prefill_ws_bytes(M, 2 * N, K);
@@ -1496,11 +1411,16 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
   if (M > 32 && shape_ok && (al & 15) == 0) {
     long ct = 0;
     bool ok = true;
+    double apart = 0;   // as one launch per matrix
     for (int p = 0; p < nmat; ++p) {
-      ct += mm_cdiv(N[p], 128);
+      const long cp = mm_cdiv(N[p], 128);
+      ct += cp;
       ok = ok && mid_ok<false>(S[p], nullptr, N[p], g);
+      const MidPlan own = plan_mid_tiles(M, cp, K);
+      const double pf = plan_prefill(M, N[p], K, g, false).us;
+      apart += own.wn != 0 ? std::min(pf, mid_us(own, M, cp, N[p], K, g, false)) : pf;
     }
-    const MidPlan mid = plan_mid_tiles(M, ct, K);
+    const MidPlan mid = choose_mid(M, ct, ntot, K, g, false, apart);
     if (ok && mid.wn != 0)
       return launch_mid<false, SK_MULTI>(mid, A, nullptr, nullptr, nullptr, nullptr, nullptr,
                                          nullptr, nullptr, 0, M, ntot, K, g, ws, ws_bytes, st, &mp);
@@ -1592,12 +1512,12 @@ extern "C" int mm_fp4_gemm_rowpacked(const uint16_t* A, const uint32_t* B, const
   }
   if (M > 32) {
     // Mid and prefill kernels reading the row-packed words in place.
-    if (const MidPlan mid = plan_mid(M, N, K);
+    if (const MidPlan mid = plan_mid(M, N, K, g, false);
         mid.wn != 0 && mid_ok<false>((const f16*)S, nullptr, N, g))
       return launch_mid<false, SK_PLAIN, true>(mid, (const f16*)A, B, (const f16*)S, nullptr,
                                                nullptr, nullptr, nullptr, (f16*)C, N, M, N, K, g,
                                                ws, ws_bytes, st);
-    const PrefillPlan p = plan_prefill(M, N, K);
+    const PrefillPlan p = plan_prefill(M, N, K, g, false);
     float* part = nullptr;
     if (p.ksplit > 1) {
       const size_t need = SK_COUNTER_BYTES + prefill_ws_bytes(M, N, K);
@@ -1724,7 +1644,7 @@ extern "C" int mm_fp4_gate_up_rowpacked(const uint16_t* A, const uint32_t* Bg, c
     // and workspace as the unfused [K, 2N] product.
     const f16 *a = (const f16*)A, *sg = (const f16*)Sg, *su = (const f16*)Su;
     hipStream_t st = (hipStream_t)stream;
-    if (const MidPlan mid = plan_mid(M, 2 * N, K);
+    if (const MidPlan mid = plan_mid(M, 2 * N, K, g, false);
         mid.wn != 0 && mid_ok<false>(sg, nullptr, N, g) && mid_ok<false>(su, nullptr, N, g)) {
       if (act)
         return launch_mid<false, SK_SWIGLU, true>(mid, a, Bg, sg, nullptr, Bu, su, nullptr,
@@ -1732,7 +1652,7 @@ extern "C" int mm_fp4_gate_up_rowpacked(const uint16_t* A, const uint32_t* Bg, c
       return launch_mid<false, SK_PAIR, true>(mid, a, Bg, sg, nullptr, Bu, su, nullptr, (f16*)C,
                                               ldc, M, N, K, g, ws, ws_bytes, st);
     }
-    const PrefillPlan p = plan_prefill(M, 2 * N, K);
+    const PrefillPlan p = plan_prefill(M, 2 * N, K, g, false);
     float* part = nullptr;
     if (p.ksplit > 1) {
       const size_t need = SK_COUNTER_BYTES + prefill_ws_bytes(M, 2 * N, K);
