@@ -23,21 +23,38 @@ extern "C" const char* mm_last_error(void) { return g_err; }
 // Bulk dequant [K/8, N] -> [K, N] fp16 (kernels_core.py:747-791; bit-exact with
 // src/marlin_gemm.metal:130-185).  Write-bound: 16 B out per packed word.
 // V adjacent words of one word row per thread.  V = 4 (N % 4 == 0, aligned
-// operands): 16-byte word loads and 8-byte stores, so a wave writes 512
-// contiguous bytes per row: 14336 x 4096 in 26.0 us (5.7 TB/s; a large copy
-// reaches 4.7 TB/s and a fill 6.9).  One word per thread (V = 1, 128 bytes per
-// wave store, the form any other N takes) took 39.5 us.  Without the
-// non-temporal hints 26.6 us.
+// operands): 16-byte word loads and 8-byte stores, 512 contiguous bytes per wave
+// and row, the threads numbered through all rows (a block per 1024 columns of each
+// row leaves a third of the threads idle at N = 1336).  One word per thread
+// (V = 1, 128 bytes per wave store) is the form any other N takes.
+// NT: the stores bypass the caches.  That is faster where a wave's rows are whole
+// 128-byte lines (N % 64 == 0, W on a line); part lines are put together in the
+// caches, where a destination that is used again may also still lie (48 MB of
+// fp16 fit them).  us with a destination never seen before and a reused one:
+//                        V = 1         V = 4         V = 4, NT
+//   4096 x 14336 FP4     32.9, 23.3    29.4, 23.7    22.8, 22.6
+//   4096 x 4096 FP4      11.7,  9.1    10.3,  8.2     7.4,  7.2
+//   5376 x 4516 INT4     19.5, 14.1    17.1, 13.0    14.6, 14.5
+//   8576 x 1336 FP4      11.3,  7.6     7.9,  7.0     7.5,  7.4
+// Non-temporal loads of the words cost 1 to 4 us in each of these.
 // ---------------------------------------------------------------------------
-template <int V, bool INT4>
+template <int V, bool INT4, bool NT = false>
 __global__ void __launch_bounds__(256)
 k_dequant(const uint32_t* __restrict__ B, const f16* __restrict__ S, const f16* __restrict__ Z,
           f16* __restrict__ W, int K, int N, int g) {
   typedef uint32_t wv __attribute__((ext_vector_type(V)));
   typedef f16 hv __attribute__((ext_vector_type(V)));
-  const int n = (blockIdx.x * 256 + threadIdx.x) * V;
-  const int kp = blockIdx.y;
-  if (n >= N) return;
+  int n, kp;
+  if constexpr (V == 1) {
+    n = blockIdx.x * 256 + threadIdx.x;
+    kp = blockIdx.y;
+    if (n >= N) return;
+  } else {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x, per_row = (uint32_t)N / V;
+    kp = (int)(i / per_row);
+    n = (int)(i - kp * per_row) * V;
+    if (kp >= K / 8) return;
+  }
   const size_t gi = (size_t)((kp * 8) / g) * N + n;
   wv w;
   hv s, z;
@@ -46,7 +63,7 @@ k_dequant(const uint32_t* __restrict__ B, const f16* __restrict__ S, const f16* 
     s[0] = S[gi];
     if constexpr (INT4) z[0] = Z[gi];
   } else {
-    w = __builtin_nontemporal_load((const wv*)(B + (size_t)kp * N + n));
+    w = *(const wv*)(B + (size_t)kp * N + n);
     s = *(const hv*)(S + gi);
     if constexpr (INT4) z = *(const hv*)(Z + gi);
   }
@@ -71,8 +88,10 @@ k_dequant(const uint32_t* __restrict__ B, const f16* __restrict__ S, const f16* 
     for (int j = 0; j < V; ++j) o[j] = v[j][i];
     if constexpr (V == 1)
       out[(size_t)i * N] = o[0];
-    else
+    else if constexpr (NT)
       __builtin_nontemporal_store(o, (hv*)(out + (size_t)i * N));
+    else
+      *(hv*)(out + (size_t)i * N) = o;
   }
 }
 
@@ -442,15 +461,20 @@ static int check_dims(const char* who, int K, int N, int g) {
 template <bool INT4>
 static int launch_dequant(const char* who, const uint32_t* B, const uint16_t* S,
                           const uint16_t* Z, uint16_t* W, int K, int N, int g, hipStream_t st) {
-  const bool v4 = N % 4 == 0 && ((uintptr_t)B & 15) == 0 &&
+  const size_t quads = (size_t)(N / 4) * (K / 8);   // of the form with four words per thread
+  const bool v4 = N % 4 == 0 && quads < ((size_t)1 << 31) && ((uintptr_t)B & 15) == 0 &&
                   (((uintptr_t)S | (uintptr_t)W | (INT4 ? (uintptr_t)Z : 0)) & 7) == 0;
-  const dim3 grid(mm_cdiv(N, v4 ? 1024 : 256), K / 8);
-  if (v4)
-    hipLaunchKernelGGL((k_dequant<4, INT4>), grid, dim3(256), 0, st, B, (const f16*)S,
-                       (const f16*)Z, (f16*)W, K, N, g);
+#define MM_LAUNCH_DEQUANT(GRID, ...)                                                             \
+  hipLaunchKernelGGL((k_dequant<__VA_ARGS__>), GRID, dim3(256), 0, st, B, (const f16*)S,          \
+                     (const f16*)Z, (f16*)W, K, N, g)
+  const dim3 grid4((unsigned)((quads + 255) / 256));
+  if (v4 && N % 64 == 0 && ((uintptr_t)W & 127) == 0)
+    MM_LAUNCH_DEQUANT(grid4, 4, INT4, true);
+  else if (v4)
+    MM_LAUNCH_DEQUANT(grid4, 4, INT4);
   else
-    hipLaunchKernelGGL((k_dequant<1, INT4>), grid, dim3(256), 0, st, B, (const f16*)S,
-                       (const f16*)Z, (f16*)W, K, N, g);
+    MM_LAUNCH_DEQUANT(dim3(mm_cdiv(N, 256), K / 8), 1, INT4);
+#undef MM_LAUNCH_DEQUANT
   MM_CHECK_LAUNCH(who);
   return 0;
 }

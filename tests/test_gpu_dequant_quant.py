@@ -217,9 +217,10 @@ def test_quantizers_edges(rng, N, K, g, dtype):
         assert np.array_equal(to_np(z), rz)
 
 
-@pytest.mark.parametrize("N", [1, 4, 255, 1020, 1028])
+@pytest.mark.parametrize("N", [1, 4, 64, 255, 576, 1020, 1028])
 def test_dequant_widths(rng, N):
-    """Four columns per thread (N % 4 == 0) and one."""
+    """Four columns per thread (N % 4 == 0), with whole lines (N % 64 == 0) and
+    without, and one."""
     import mmfp4
     K, g = 64, 32
     packed = rng.integers(0, 2**32, (K // 8, N), dtype=np.uint64).astype(np.uint32)
@@ -251,3 +252,34 @@ def test_quantize_fp4_wide_float32_groups(rng, e):
     packed, s = mmfp4.quantize_fp4(to_dev(w), group_size=g)
     assert np.array_equal(to_np(s).view(np.uint16), rs.view(np.uint16))
     assert np.array_equal(to_np(packed).view(np.uint32), rp)
+
+
+def test_dequant_wide_form_is_not_slower():
+    """Four words per thread against one (scales that are not 8-byte aligned) into a
+    destination that is used again, at a width whose rows end inside a cache line:
+    13.0 against 14.1 us; 16.4 with stores that bypassed the caches."""
+    import mmfp4
+    K, N, g = 5376, 4516, 32
+    p = torch.randint(-2**31, 2**31 - 1, (K // 8, N), device="cuda", dtype=torch.int32)
+    s = torch.full((K // g * N + 4,), 0.01, device="cuda", dtype=torch.float16)
+    z = torch.full((K // g, N), 7.0, device="cuda", dtype=torch.float16)
+    out = torch.empty((K, N), device="cuda", dtype=torch.float16)
+    lib = mmfp4._lib
+
+    def us(first):
+        sv = s[first:first + K // g * N]
+        times = []
+        for _ in range(8):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(50):
+                lib.call("mm_u4_dequant", lib.ptr(p), lib.ptr(sv), lib.ptr(z), lib.ptr(out), K, N,
+                         g, lib.stream_of(out))
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 20)
+        return min(times)
+
+    announce(f"dequant forms K={K} N={N}")
+    one, four = us(1), us(0)
+    assert four < 1.05 * one, f"{four:.2f} us with four words per thread, {one:.2f} with one"
