@@ -1425,10 +1425,10 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
       return launch_mid<false, SK_MULTI>(mid, A, nullptr, nullptr, nullptr, nullptr, nullptr,
                                          nullptr, nullptr, 0, M, ntot, K, g, ws, ws_bytes, st, &mp);
   }
-  if (!off32 || M > 32 || !shape_ok ||
+  if (!off32 || M > 32 || !shape_ok || (M > 16 && tiles > SK_MAX_TILES) ||
       flush_steps(g, M <= 16 ? sk_spw<1>() : sk_spw<2>()) == 0) {
-    // One product per launch (larger M, or shapes the GEMM entry rejects with
-    // its own message).
+    // One product per launch (larger M, more columns than one launch has counters
+    // for, or shapes the GEMM entry rejects with its own message).
     for (int p = 0; p < nmat; ++p) {
       const int rc = gemm_dispatch<false>(who, A, B[p], S[p], nullptr, C[p], M, N[p], K, g, ws,
                                           ws_bytes, st);

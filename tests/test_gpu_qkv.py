@@ -58,6 +58,21 @@ def test_fused_qkv_1d_input_vs_oracle(rng):
         assert max_abs_rel(to_np(o), ref) <= TOL
 
 
+def test_fused_qkv_more_columns_than_one_launch_takes():
+    """17..32 rows, over a million columns together but not each: as three products."""
+    import mmfp4
+    M, K, N, g = 20, 64, 400_000, 64
+    gen = torch.Generator("cuda").manual_seed(5)
+    mats = [(torch.randint(-2**31, 2**31 - 1, (K // 8, N), device="cuda", dtype=torch.int32,
+                           generator=gen),
+             (torch.rand(1, N, device="cuda", generator=gen) * 0.01).half()) for _ in range(3)]
+    x = torch.randn(M, K, device="cuda", generator=gen).half()
+    announce(f"fused qkv M={M} N=3 x {N}")
+    outs = mmfp4.mmfp4_fused_qkv(x, *[t for m in mats for t in m], g)
+    for o, m in zip(outs, mats):
+        assert torch.equal(o, mmfp4.marlin_gemm_fp4(x, *m, g))
+
+
 def test_fused_qkv_errors():
     import mmfp4
     x = torch.zeros((1, 64), dtype=torch.float16, device="cuda")
