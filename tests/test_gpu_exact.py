@@ -15,9 +15,11 @@ Each case is chosen to land on one kernel family (the selection rules of
 gemm_dispatch / pair_dispatch / mm_moe_grouped_gemm):
   k_skinny_dual  M <= 8 narrow layers;  k_strip  8 < M <= 16, K*N <= 4096^2;
   k_skinny       M <= 16 wide (no split) and split-K (14336 -> 4096), MT=2 for
-                 17..32 rows;  k_prefill2 M > 32 with K % 64 == 0 (and its
-                 split-K reduce when the grid is small);  k_prefill  N % 8 != 0
-                 or K % 64 != 0;  row-packed and [N, K/g]-scale variants;
+                 17..32 rows;  k_mid  M > 32 until the prefill tiles are faster
+                 (K % 128 == 0, g % 32 == 0, N % 8 == 0);  k_prefill2  above, with
+                 K % 64 == 0 (and its split-K reduce when the grid is small);
+                 k_prefill  N % 8 != 0 or K % 64 != 0;  row-packed and
+                 [N, K/g]-scale variants;
                  multi (QKV); gate/up pair (act=0, no SwiGLU rounding);
                  k_moe_grouped and k_moe_prefill.
 """
@@ -336,6 +338,49 @@ def test_mid_bit_exact(rng, M, K, N, g):
     q, sc, z = _exact_u4(rng, K, N, g)
     announce(f"exact mid u4 M={M} K={K} N={N} g={g}")
     _same(mmfp4.marlin_gemm_int4(td[0], to_dev(q), to_dev(sc), to_dev(z), g),
+          ofp4.gemm_u4_ref(a, q, sc, z, g))
+
+
+@pytest.mark.parametrize("M,K,N,g", [(65, 512, 8200, 128), (100, 640, 8264, 64),
+                                     (128, 640, 8200, 32), (97, 1024, 8264, 256)])
+def test_mid_128_row_tiles(rng, M, K, N, g):
+    """65..128 rows with more 64-row tiles than CUs take 128-row tiles: plain, pair,
+    SwiGLU and QKV forms, Marlin and row-packed, widths that end inside a tile."""
+    import mmfp4
+    a = _acts(rng, M, K)
+    w = [_exact_fp4(rng, K, N, g) for _ in range(2)]
+    # the sums are exact in fp32; only results are rounded
+    sums = [a.astype(np.float32) @ ofp4.dequant_fp4_f32(p, s, g) for p, s in w]
+    both = np.concatenate(sums, 1).astype(np.float16)
+    gate, up = (torch.from_numpy(x).double() for x in sums)
+    swiglu = torch.nn.functional.silu(gate) * up
+    announce(f"exact mid 128-row tiles M={M} K={K} N={N} g={g}")
+    x, (pg, sg), (pu, su) = to_dev(a), *[[to_dev(t) for t in m] for m in w]
+    _same(mmfp4.fused_gate_up_gemm(x, pg, sg, pu, su, g), both)
+    outs = [mmfp4.mmfp4_fused_gate_up_marlin(x, pg, sg, pu, su, g)]
+    # the same matrices as one of 2 N columns, and as three in one launch
+    p2, s2 = torch.cat([pg, pu], 1).contiguous(), torch.cat([sg, su], 1).contiguous()
+    _same(mmfp4.marlin_gemm_fp4(x, p2, s2, g), both)
+    n = 72
+    qkv = mmfp4.mmfp4_fused_qkv(x, p2, s2, pg[:, :8].contiguous(), sg[:, :8].contiguous(),
+                                pu[:, :n].contiguous(), su[:, :n].contiguous(), g)
+    for o, r in zip(qkv, (both, both[:, :8], both[:, N:N + n]), strict=True):
+        _same(o, r)
+    if g % 64 == 0:
+        rg, ru = pg.t().contiguous(), pu.t().contiguous()
+        _same(mmfp4.mmfp4_gemm_rowpacked(x, p2.t().contiguous(), s2, g), both)
+        outs.append(mmfp4.mmfp4_fused_gate_up(x, rg, sg, ru, su, g))
+        lib, out = mmfp4._lib, torch.empty((M, 2 * N), dtype=torch.float16, device="cuda")
+        ws = lib.workspace(out.device, int(lib.load().mm_gemm_workspace_bytes(M, 2 * N, K)))
+        lib.call("mm_fp4_gate_up_rowpacked", *map(lib.ptr, (x, rg, sg, ru, su, out)), M, N, K, g,
+                 0, lib.ptr(ws), ws.numel(), lib.stream_of(out))
+        _same(out, both)
+    # one fp16 rounding (2^-11; below 2^-14 2^-25) of the product; its own error is that
+    # of exp(-gate) at most, |gate| 2^-23 with |gate| < 20 where the result is normal
+    for out in outs:
+        assert torch.allclose(out.double().cpu(), swiglu, rtol=2**-11 + 2**-18, atol=2**-24)
+    q, sc, z = _exact_u4(rng, K, 2 * N, g)
+    _same(mmfp4.marlin_gemm_int4(x, to_dev(q), to_dev(sc), to_dev(z), g),
           ofp4.gemm_u4_ref(a, q, sc, z, g))
 
 
