@@ -1,5 +1,5 @@
 """GPU parity of the fused QKV projection (one launch over the Q, K and V
-matrices' column tiles for M <= 16) against the fp32 reference built from
+matrices' column tiles at decode and mid sizes) against the fp32 reference built from
 the bit-exact dequant, plus the oracle on a small ragged case."""
 
 from __future__ import annotations
@@ -107,6 +107,18 @@ def test_binding_and_ctypes_agree(monkeypatch, M):
         yield mmfp4.mmfp4_gemm_rowpacked(x, rows[0], rows[1].t().contiguous(), g)
 
     announce(f"binding against ctypes M={M}")
+    # the binding is there, takes the plain operands and leaves the others
+    assert kernels._binding()
+    bad = (x.float(), x.t().contiguous().t()) if M > 1 else (x.float(),)
+    for args, plain in [((x, *odd[:4]), False), ((x, *marlin[:4]), True)] + \
+            [((b, *marlin[:4]), False) for b in bad]:
+        b, w0, s0, w1, s1 = args
+        r0, r1 = w0.t().contiguous(), w1.t().contiguous()
+        took = [kernels._fast("qkv", b, (w0, w1, w0), (s0, s1, s0), g),
+                kernels._fast("gate_up", b, w0, s0, w1, s1, g, False, True),
+                kernels._fast("gate_up", b, r0, s0, r1, s1, g, True, True),
+                kernels._fast("rowpacked", b, r0, s0, g)]
+        assert [t is not None for t in took] == [plain] * 4
     fast = list(calls())
     monkeypatch.setattr(kernels, "_BINDING", False)
     for a, b in zip(fast, calls(), strict=True):
