@@ -66,7 +66,7 @@ struct MidShape {
 // column group wn, LDS column 64*wn + 2*l32 + j (TM: 64*wn + 32*j + l32), as
 // pf2_mainloop; `src` as there.  G128: g % 128 == 0 (a chunk lies in one group);
 // otherwise g % 32 == 0 (a wave's share of a chunk does).  Requires K % 128 == 0.
-template <bool INT4, int RB, int WN, bool G128, bool TM, int RBL = RB, class Src>
+template <bool INT4, int RB, int WN, bool G128, bool TM, class Src>
 MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, char* smem,
                          f32x16 (&acc)[RB][2]) {
   using Sh = MidShape<INT4, RB, WN>;
@@ -77,7 +77,7 @@ MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
   const int wn = wave % WN, wk = wave / WN;
   const int l32 = lane & 31, h = lane >> 5;
   const int ngroups = K / g, ld = src.ld;
-  auto asw = [](int r) { return PPR == 8 ? (r >> 1) & 7 : r & 15; };
+  auto asw = [](int r) { return r & 15; };
 
   const f16* a_src[Sh::A_IT];
 #pragma unroll
@@ -182,7 +182,7 @@ MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
       wv[0] = w.x, wv[1] = w.y;
     }
 #pragma unroll
-    for (int rb = 0; rb < RBL; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
       af[slot][rb] =
           *(const f16x8*)(base + a_base + rb * 32 * BK * 2 +
                           (((ROWP ? 4 * wk + 2 * h + s : 2 * t + h) ^ asx) * 16));
@@ -218,13 +218,13 @@ MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
   };
   auto mfma = [&](int slot) {
 #pragma unroll
-    for (int rb = 0; rb < RBL; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int j = 0; j < CW; ++j)
         acc[rb][j] =
             __builtin_amdgcn_mfma_f32_32x32x16_f16(af[slot][rb], bq[slot][j], acc[rb][j], 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < RBL * CW; ++i) {
+    for (int i = 0; i < RB * CW; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
       __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // DS read
       __builtin_amdgcn_sched_group_barrier(0x002, 9, 0);   // VALU
@@ -240,28 +240,22 @@ MM_DEV void mid_mainloop(const Src& src, int K, int g, int c_beg, int c_end, cha
     asm volatile("" ::: "memory");
   };
   next_chunk();
-  if constexpr (RBL > 0) {
-    read(0, 0, 0);
-    read_scale(0, c_beg * BK);
-    decode(0);
-  }
+  read(0, 0, 0);
+  read_scale(0, c_beg * BK);
+  decode(0);
   auto chunk = [&](int ch, auto stc) {
     constexpr int st = decltype(stc)::value, sn = (st + 1) % NST;
     // The stage of chunk ch - 1 was read by every wave before the last barrier.
     issue(min(ch + NST - 1, last), (st + NST - 1) % NST);
     static_assert(STEPS == 2, "one operand slot per step");
-    if constexpr (RBL > 0) {
-      read(st, 1, 1);
-      mfma(0);
-      decode(1);
-    }
+    read(st, 1, 1);
+    mfma(0);
+    decode(1);
     next_chunk();
-    if constexpr (RBL > 0) {
-      read(sn, 0, 0);
-      read_scale(sn, min(ch + 1, last) * BK);
-      mfma(1);
-      decode(0);
-    }
+    read(sn, 0, 0);
+    read_scale(sn, min(ch + 1, last) * BK);
+    mfma(1);
+    decode(0);
   };
   for (int ch = c_beg; ch < c_end; ch += NST) {
     static_for(
