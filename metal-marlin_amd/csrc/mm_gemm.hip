@@ -13,8 +13,8 @@
 //    block holds NW waves that split its K range; the block reduces the waves
 //    in LDS, and a K split across blocks is reduced by the last-arriving block
 //    (deterministic order, counter left at zero for the next call).
-//  * mid (M > 32, until the prefill tiles fill the chip): 64- or 128-row tiles
-//    whose waves split K (mm_mid.h).
+//  * mid (M > 32, until the prefill tiles are faster: mm_plan.h): 64- or 128-row
+//    tiles whose waves split K (mm_mid.h).
 //  * prefill: 32x32x16 MFMA tiles of 256 columns over an LDS ring (mm_prefill.h;
 //    k_prefill for shapes outside its 8-column and 64-k pieces).
 #include <algorithm>
@@ -71,9 +71,9 @@ struct SkMulti {
 // fp32 with PW = N, 2N for the pair modes (gate at n, up at N + n), or ntot.
 // ROWP: 0 Marlin-layout weights; 1, 2 row-packed [N, K/8] weights with
 // scales [N, K/g] (1) or [K/g, N] (2), transposed through LDS into the
-// Marlin operand order (skinny_wave RT) or, the pair with groups of 128 k or
-// more, read in place from LDS (skinny_wave_rows); 3 Marlin-layout weights with scales
-// [N, K/g].
+// Marlin operand order (skinny_wave RT) or, the pair at up to 16 rows with groups
+// of 128 or a multiple of 256 k, read in place from LDS (skinny_wave_rows);
+// 3 Marlin-layout weights with scales [N, K/g].
 // Row-packed single-tile blocks: the RT staging takes a few registers over
 // the 128 that keep two 8-wave blocks resident per CU; at that limit the
 // flush intervals listed here compile without spills (the others keep the
@@ -676,10 +676,10 @@ k_prefill2(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
 
 // ===========================================================================
 // Mid-sized path (main loop in mm_mid.h): M > 32 up to the sizes where the
-// 256-column prefill tiles fill the chip.  grid = (column tiles, row tiles, K
-// splits).  A K split hands its sums over as k_skinny's does (sc1 partials,
-// an arrival counter per tile, the last block adds the splits in split order):
-// a separate reduction launch costs about 5 us, a quarter of these calls.
+// 256-column prefill tiles are faster (mm_plan.h).  grid = (column tiles, row
+// tiles, K splits).  A K split hands its sums over as k_skinny's does (sc1
+// partials, an arrival counter per tile, the last block adds the splits in split
+// order): a separate reduction launch costs about 5 us, a quarter of these calls.
 // ===========================================================================
 // ROWS: B (and B2) are row-packed [N, K/8] FP4 words.
 template <bool INT4, int RB, int WN, bool G128, int ACT, bool ROWS = false>

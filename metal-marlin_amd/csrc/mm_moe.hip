@@ -541,8 +541,8 @@ k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
   // launch has one to two rounds of tiles, and in expert order the CUs that got
   // a full tile last kept the launch going while the others were idle (CUs busy
   // 63% of the launch, 82% of a dense one).  Qwen3-30B-A3B shapes with uneven
-// loads, mean of gate_up and down at T = 1024: 77.5 -> 70.7 us; T = 512, 2048 and
-// 4096 within 2%.
+  // loads, mean of gate_up and down at T = 1024: 77.5 -> 70.7 us; T = 512, 2048
+  // and 4096 within 2%.
   if (wave < RB) {
     int* const t = tp + wave * (E + 1);
     int base = 0;

@@ -405,7 +405,7 @@ MM_DEV void skinny_wave(const f16* __restrict__ A, int lda, const int* __restric
 }
 
 // skinny_wave for the row-packed FP4 pair (two tiles, up to 16 rows, SPW == 8,
-// FL >= 4: groups of 128 k or more).  A round's words -- 8 16-byte pieces of 4
+// FL >= 4: groups of 128 k or a multiple of 256).  A round's words -- 8 16-byte pieces of 4
 // words per column -- go global -> LDS directly, with whole row segments, into
 // the wave's region `stage` (8 KiB per tile, the wave's own: no barrier), and a
 // lane reads its columns' words back a piece at a time.  Which words of a

@@ -182,8 +182,8 @@ def marlin_gemm_fp4(A: torch.Tensor, B_packed: torch.Tensor, scales: torch.Tenso
 
     A [*, K] (any float dtype, computed as fp16), B_packed [K/8, N] int32/uint32
     Marlin layout, scales [K/group_size, N].  Returns fp16 [*, N].  M <= 32 runs
-    the decode kernel, larger M the MFMA prefill kernel (metal_dispatch.py:
-    4083-4098 chooses by M the same way).
+    the decode kernels, larger M the MFMA mid-sized or prefill kernel, whichever is
+    faster (metal_dispatch.py:4083-4098 chooses by M too).
     """
     return _gemm("fp4", A, B_packed, scales, None, group_size)
 
@@ -211,9 +211,9 @@ def mmfp4_gemm_rowpacked(A: torch.Tensor, B_rows: torch.Tensor, scales: torch.Te
     """A [M, K] @ dequant(B_rows)^T with row-packed weights read in place:
     B_rows [N, K/8] words, scales [K/group_size, N] (the layer's canonical
     layout) or [N, K/group_size] (layers/mmfp4_linear.py:549-598).  M <= 32
-    runs the decode kernels; larger M the pipelined prefill kernel, which
-    reads the words in place too but takes [K/group_size, N] scales (the
-    other layout is transposed here, K/group_size x N halves)."""
+    runs the decode kernels; larger M the mid-sized or the pipelined prefill
+    kernel, which read the words in place too but take [K/group_size, N] scales
+    (the other layout is transposed here, K/group_size x N halves)."""
     if isinstance(A, torch.Tensor) and A.dim() == 2 and B_rows.dim() == 2 and \
             scales.dim() == 2 and scales.shape[1] == B_rows.shape[0]:
         out = _fast("rowpacked", A, B_rows, scales, group_size)
@@ -325,7 +325,7 @@ def mmfp4_fused_gate_up(x: torch.Tensor, gate_packed: torch.Tensor, gate_scales:
     With N % 8 == 0 and a group size that is a multiple of 32 (up to 32 rows)
     or of 64 (above) the row-packed words are read in place at every M
     (mm_fp4_gate_up_rowpacked: the decode kernel up to 32 rows, the
-    pipelined prefill kernel above); other shapes
+    mid-sized or the pipelined prefill kernel above); other shapes
     are transposed to the Marlin layout on the device for each call (as the
     reference's own M < 64 path does); callers that keep the Marlin layout
     call `mmfp4_fused_gate_up_marlin`.

@@ -6,9 +6,9 @@ word (n, j) holding inputs 8j..8j+7 of output n (LSB first); scales are
 [n_groups, out_features] or [out_features, n_groups].  Both the functional
 `mmfp4_gemm` and `MMFP4Linear` read the row-packed words in place
 (mm_fp4_gemm_rowpacked): the decode kernels up to 32 rows (group size a
-multiple of 32), the pipelined prefill kernel above (group size a multiple
-of 64, out_features % 8 == 0), so the layer holds one copy of its weights.  Other shapes run the Marlin-layout kernels
-on [in // 8, out] words: the functional form converts per call (as the
+multiple of 32), the mid-sized or the pipelined prefill kernel above (group size
+a multiple of 64, out_features % 8 == 0), so the layer holds one copy of its
+weights.  Other shapes run the Marlin-layout kernels on [in // 8, out] words: the functional form converts per call (as the
 reference does on every call); the layer converts once on the device and
 keeps the copy as a non-persistent buffer (the reference's
 `_kernel_packed_weights`), rebuilt whenever `packed_weights` is written or
