@@ -80,10 +80,10 @@ DENSE = [
     (12, 4096, 28672, 64, "k_skinny MT=1, 128-column blocks"),
     (32, 4096, 6144, 128, "k_skinny MT=2 split-K, 64-column blocks"),
     (32, 14336, 4096, 128, "k_skinny MT=2 split-K"),
-    (64, 4096, 1024, 128, "k_prefill2 64-row tile"),
-    (128, 14336, 4096, 128, "k_prefill2 split-K + reduce"),
-    (512, 4096, 14336, 128, "k_prefill2 (cfg4 M=512)"),
-    (300, 2048, 1000, 64, "k_prefill2 ragged"),
+    (64, 4096, 1024, 128, "k_mid, 64 columns, split-K"),
+    (128, 14336, 4096, 128, "k_mid split-K"),
+    (512, 4096, 14336, 128, "config 4 up M=512"),
+    (300, 2048, 1000, 64, "k_mid ragged"),
     (100, 520, 260, 8, "k_prefill (N % 8, K % 64)"),
     (40, 200, 96, 8, "k_prefill (K % 64)"),
     # every tile shape bench.py times, at its full size: config 2 (M = 8, 32)
@@ -157,9 +157,9 @@ def test_fp4_gemm_bit_exact_m8192_rows(rng, K, N):
 def test_rowpacked_and_mmfp4_bit_exact(rng, M, K, N, g):
     """Row-packed words (both scale layouts) and Marlin words with [N, K/g]
     scales: the two-slab and skinny in-place variants (M <= 32, one and two
-    row blocks, split-K) and the pipelined prefill kernel on row-packed words
-    (M > 32: 64-, 128- and 256-row tiles, split-K, ragged N), and K % 256 != 0
-    (rounds overhanging K) on both."""
+    row blocks, split-K), the mid-sized kernel and the pipelined prefill kernel on
+    row-packed words (M > 32: split-K, ragged N), and K % 256 != 0 (rounds
+    overhanging K)."""
     import mmfp4
     packed, scales = _exact_fp4(rng, K, N, g)
     a = _acts(rng, M, K)
@@ -338,6 +338,31 @@ def test_mid_bit_exact(rng, M, K, N, g):
     q, sc, z = _exact_u4(rng, K, N, g)
     announce(f"exact mid u4 M={M} K={K} N={N} g={g}")
     _same(mmfp4.marlin_gemm_int4(td[0], to_dev(q), to_dev(sc), to_dev(z), g),
+          ofp4.gemm_u4_ref(a, q, sc, z, g))
+
+
+@pytest.mark.parametrize("M,K,N,g", [(40, 4160, 520, 64), (64, 1088, 256, 64),
+                                     (100, 4160, 1032, 64), (200, 2112, 520, 64)])
+def test_prefill_split_bit_exact(rng, M, K, N, g):
+    """The 64- and 128-row prefill tiles and their split of K, which K % 128 == 0 no
+    longer reaches up to a few hundred rows: plain, pair, row-packed and INT4."""
+    import mmfp4
+    a = _acts(rng, M, K)
+    w = [_exact_fp4(rng, K, N, g) for _ in range(2)]
+    both = np.concatenate([ofp4.gemm_fp4_ref(a, p, s, g) for p, s in w], 1)
+    announce(f"exact prefill split M={M} K={K} N={N} g={g}")
+    x, (pg, sg), (pu, su) = to_dev(a), *[[to_dev(t) for t in m] for m in w]
+    rg, ru = pg.t().contiguous(), pu.t().contiguous()
+    _same(mmfp4.marlin_gemm_fp4(x, pg, sg, g), both[:, :N])
+    _same(mmfp4.mmfp4_gemm_rowpacked(x, rg, sg, g), both[:, :N])
+    _same(mmfp4.fused_gate_up_gemm(x, pg, sg, pu, su, g), both)
+    lib, out = mmfp4._lib, torch.empty((M, 2 * N), dtype=torch.float16, device="cuda")
+    ws = lib.workspace(out.device, int(lib.load().mm_gemm_workspace_bytes(M, 2 * N, K)))
+    lib.call("mm_fp4_gate_up_rowpacked", *map(lib.ptr, (x, rg, sg, ru, su, out)), M, N, K, g, 0,
+             lib.ptr(ws), ws.numel(), lib.stream_of(out))
+    _same(out, both)
+    q, sc, z = _exact_u4(rng, K, N, g)
+    _same(mmfp4.marlin_gemm_int4(x, to_dev(q), to_dev(sc), to_dev(z), g),
           ofp4.gemm_u4_ref(a, q, sc, z, g))
 
 

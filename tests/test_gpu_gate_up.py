@@ -1,7 +1,7 @@
 """GPU parity of the fused gate/up operator (one launch over the gate and up
 matrices): silu(x @ Wg) * (x @ Wu) and [x @ Wg | x @ Wu], against the fp32
-reference built from the bit-exact dequant, on both kernels (decode M <= 32,
-prefill M > 32), with and without a K split, and against the oracle on a
+reference built from the bit-exact dequant, on the decode (M <= 32), mid-sized
+and prefill kernels (M > 32), with and without a K split, and against the oracle on a
 small case."""
 
 from __future__ import annotations
@@ -59,7 +59,7 @@ def test_gate_up_vs_fp32_reference(M, K, N, g):
 def test_gate_up_rowpacked_vs_oracle(rng, M, K, N, g):
     """mmfp4_fused_gate_up on row-packed [N, K/8] weights (the reference's
     documented layout) against the numpy oracle: read in place by the decode
-    kernel (M <= 16) and the pipelined prefill kernel (M > 16, including a
+    kernel (M <= 32) and the mid-sized and prefill kernels (M > 32, including a
     ragged N, a split-K grid and K % 256 != 0); g=32 is read in place up to
     32 rows and transposed per call above."""
     import mmfp4

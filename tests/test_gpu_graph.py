@@ -4,8 +4,9 @@ The library's launches take the caller's stream and allocate nothing once a
 stream's workspace exists, and the split-K arrival counters are returned to
 zero by the last block of each tile (no memset node).  So a caller can
 capture them: the four Llama-layer GEMMs (two-slab, skinny and split-K
-hand-off at M=1; the pipelined prefill kernel with and without its K split
-at M=128) and the MoE MLP (sort, grouped GEMMs, combine; decode- and
+hand-off at M=1; the mid-sized kernel at M=128, and the pipelined prefill
+kernel, with and without its K split, where K is no multiple of 128) and the
+MoE MLP (sort, grouped GEMMs, combine; decode- and
 prefill-sized groups), and the row-packed GEMM and gate/up pair, are
 captured once and replayed several times, with new inputs copied into the
 captured buffers and eager launches of the same entry points in between.  Every replay must equal the eager result on the
@@ -24,7 +25,7 @@ G = 128
 LAYER = [(4096, 6144), (4096, 4096), (4096, 14336), (14336, 4096)]
 
 
-def _words(gen, K, N):
+def _words(gen, K, N, G=G):
     p = torch.randint(-2**31, 2**31 - 1, (K // 8, N), generator=gen, dtype=torch.int32,
                       device="cuda")
     s = (torch.rand((K // G, N), generator=gen, device="cuda") * 0.01 + 1e-3).half()
@@ -47,32 +48,33 @@ def _capture(fn, warmup=2):
     return g, outs
 
 
-@pytest.mark.parametrize("M", [1, 128])
-def test_layer_gemms_graph_replay(M):
+@pytest.mark.parametrize("M,shapes,g", [(1, LAYER, 128), (128, LAYER, 128),
+                                        (128, [(4160, 4096), (960, 14336)], 64)])
+def test_layer_gemms_graph_replay(M, shapes, g):
     import mmfp4
     gen = torch.Generator(device="cuda").manual_seed(11 + M)
-    ws = [_words(gen, K, N) for K, N in LAYER]
-    xs = {K: torch.empty((M, K), dtype=torch.float16, device="cuda") for K, _ in LAYER}
+    ws = [_words(gen, K, N, g) for K, N in shapes]
+    xs = {K: torch.empty((M, K), dtype=torch.float16, device="cuda") for K, _ in shapes}
 
     def layer():
-        return [mmfp4.marlin_gemm_fp4(xs[K], w[0], w[1], G) for (K, _), w in zip(LAYER, ws)]
+        return [mmfp4.marlin_gemm_fp4(xs[K], w[0], w[1], g) for (K, _), w in zip(shapes, ws)]
 
     for x in xs.values():
         x.copy_(torch.randn(x.shape, generator=gen, device="cuda").half())
-    announce(f"graph capture of the layer GEMMs M={M}")
-    g, outs = _capture(layer)
+    announce(f"graph capture of the layer GEMMs M={M} {shapes}")
+    graph, outs = _capture(layer)
     for rep in range(4):
         for x in xs.values():
             x.copy_(torch.randn(x.shape, generator=gen, device="cuda").half())
         torch.cuda.synchronize()
         ref = layer()                                   # eager, same inputs
         torch.cuda.synchronize()
-        g.replay()
+        graph.replay()
         torch.cuda.synchronize()
-        for (K, N), o, r in zip(LAYER, outs, ref):
+        for (K, N), o, r in zip(shapes, outs, ref):
             assert torch.equal(o.view(torch.int16), r.view(torch.int16)), (rep, K, N)
         # unrelated eager work on the same entry point between replays
-        mmfp4.marlin_gemm_fp4(xs[4096][:1], ws[1][0], ws[1][1], G)
+        mmfp4.marlin_gemm_fp4(xs[shapes[1][0]][:1], ws[1][0], ws[1][1], g)
 
 
 @pytest.mark.parametrize("T,E,k", [(32, 16, 4), (512, 16, 4), (1024, 16, 4)])

@@ -81,7 +81,7 @@ def test_rowpacked_gemm_in_place(M, K, N, g):
     either layout the layer accepts ([K/g, N] canonical, [N, K/g] transposed)
     (layers/mmfp4_linear.py:549-598 without its per-call transpose): parity
     with the fp32 reference of the same weights, including the split-K shape
-    14336 -> 4096, and above 16 rows the pipelined prefill kernel on the same
+    14336 -> 4096, and above 32 rows the mid-sized or prefill kernel on the same
     words.  Both scale layouts give bit-identical results."""
     import mmfp4
     gen = torch.Generator(device="cuda").manual_seed(M * 3 + K + N)
