@@ -335,12 +335,12 @@ MM_DEV uint32_t fp4_pair(uint32_t word, float v0, float v1) {
                                                   BYTE);
 }
 
-constexpr int QT_N = 64;      // rows of W (columns of the packed matrix) per block
 constexpr int QT_WORDS = 64;  // words (8 k) per row and block: one wave-wide load
 constexpr int QT_WAVES = 4;
-constexpr int QT_ROWS = 4;    // rows a wave loads together
 
-template <typename T, bool INT4>
+// QT_N: rows of W (columns of the packed matrix) per block; QT_ROWS: rows a wave
+// loads together.
+template <typename T, bool INT4, int QT_N, int QT_ROWS>
 __global__ void __launch_bounds__(QT_WAVES * 64)
 k_quantize_tile(const T* __restrict__ Wt, int N, int K, int g, uint32_t* __restrict__ B,
                 f16* __restrict__ S, f16* __restrict__ Z) {
@@ -430,14 +430,15 @@ k_quantize_tile(const T* __restrict__ Wt, int N, int K, int g, uint32_t* __restr
     }
   }
   __syncthreads();
-  const int n = n0 + lane;
+  constexpr int WSTEP = QT_WAVES * 64 / QT_N;
+  const int col = threadIdx.x % QT_N, n = n0 + col;
   if (n >= N) return;
-  for (int w = wave; w < QT_WORDS && w0 + w < KP; w += QT_WAVES)
-    B[(size_t)(w0 + w) * N + n] = words[w][lane];
-  for (int q = wave; q < QT_WORDS / wpg && w0 + q * wpg < KP; q += QT_WAVES) {
+  for (int w = threadIdx.x / QT_N; w < QT_WORDS && w0 + w < KP; w += WSTEP)
+    B[(size_t)(w0 + w) * N + n] = words[w][col];
+  for (int q = threadIdx.x / QT_N; q < QT_WORDS / wpg && w0 + q * wpg < KP; q += WSTEP) {
     const size_t at = (size_t)(w0 / wpg + q) * N + n;
-    S[at] = sc[q][lane];
-    if constexpr (INT4) Z[at] = zp[q][lane];
+    S[at] = sc[q][col];
+    if constexpr (INT4) Z[at] = zp[q][col];
   }
 }
 
@@ -491,17 +492,34 @@ extern "C" int mm_u4_dequant(const uint32_t* B, const uint16_t* S, const uint16_
   return launch_dequant<true>("mm_u4_dequant", B, S, Z, W, K, N, g, (hipStream_t)stream);
 }
 
+// Rows per block: a block of 64 rows works through four batches of rows in turn
+// (8 to 13 us alone), which leaves most CUs idle while there are fewer of them than
+// CUs; blocks of 4 rows then take one batch.  us, per-group kernel, 64 rows, 4 rows:
+// INT4 33 x 1024 g = 8 2.6, 9.0, 2.4; 256 x 256 g = 32 7.3, 9.2, 2.5; FP4 (fp16)
+// 1000 x 4096 g = 128 57, 12.0, 5.7; 512 x 14336 68, 12.3, 7.8; but float32
+// 4096 x 4096 g = 64 161, 17.8, 19.5 (16-byte runs of output).
+template <typename T, bool INT4>
+static void launch_quantize_tile(const void* W, int N, int K, int g, uint32_t* B, uint16_t* S,
+                                 uint16_t* Z, hipStream_t st) {
+#define MM_LAUNCH_QT(QN, QR)                                                                     \
+  hipLaunchKernelGGL((k_quantize_tile<T, INT4, QN, QR>),                                         \
+                     dim3(mm_cdiv(N, QN), mm_cdiv(K / 8, QT_WORDS)), dim3(QT_WAVES * 64), 0, st,  \
+                     (const T*)W, N, K, g, B, (f16*)S, (f16*)Z)
+  if ((long)mm_cdiv(N, 64) * mm_cdiv(K / 8, QT_WORDS) < 256)
+    MM_LAUNCH_QT(4, 1);
+  else
+    MM_LAUNCH_QT(64, 4);
+#undef MM_LAUNCH_QT
+}
+
 extern "C" int mm_fp4_quantize(const void* W, int w_is_f32, int N, int K, int g, uint32_t* B,
                                uint16_t* S, void* stream) {
   if (int rc = check_dims("mm_fp4_quantize", K, N, g)) return rc;
   if (quant_tile_ok(W, g)) {
-    const dim3 tiles(mm_cdiv(N, QT_N), mm_cdiv(K / 8, QT_WORDS));
     if (w_is_f32)
-      hipLaunchKernelGGL((k_quantize_tile<float, false>), tiles, dim3(QT_WAVES * 64), 0,
-                         (hipStream_t)stream, (const float*)W, N, K, g, B, (f16*)S, nullptr);
+      launch_quantize_tile<float, false>(W, N, K, g, B, S, nullptr, (hipStream_t)stream);
     else
-      hipLaunchKernelGGL((k_quantize_tile<f16, false>), tiles, dim3(QT_WAVES * 64), 0,
-                         (hipStream_t)stream, (const f16*)W, N, K, g, B, (f16*)S, nullptr);
+      launch_quantize_tile<f16, false>(W, N, K, g, B, S, nullptr, (hipStream_t)stream);
     MM_CHECK_LAUNCH("mm_fp4_quantize");
     return 0;
   }
@@ -541,9 +559,7 @@ extern "C" int mm_u4_quantize(const uint16_t* W, int N, int K, int g, uint32_t* 
                               uint16_t* Z, void* stream) {
   if (int rc = check_dims("mm_u4_quantize", K, N, g)) return rc;
   if (quant_tile_ok(W, g)) {
-    hipLaunchKernelGGL((k_quantize_tile<f16, true>),
-                       dim3(mm_cdiv(N, QT_N), mm_cdiv(K / 8, QT_WORDS)), dim3(QT_WAVES * 64), 0,
-                       (hipStream_t)stream, (const f16*)W, N, K, g, B, (f16*)S, (f16*)Z);
+    launch_quantize_tile<f16, true>(W, N, K, g, B, S, Z, (hipStream_t)stream);
     MM_CHECK_LAUNCH("mm_u4_quantize");
     return 0;
   }

@@ -192,9 +192,12 @@ def _crafted(rng, n, k, dtype):
 # 8 * 2^i up to 512 run the tiled quantizer; 24 and 1024 the per-group one.
 @pytest.mark.parametrize("N,K,g", [(1, 8, 8), (63, 512, 16), (65, 520, 8), (64, 1536, 512),
                                    (130, 1152, 128), (66, 544, 32), (33, 768, 256),
-                                   (70, 576, 64), (40, 72, 24), (9, 2048, 1024)])
+                                   (70, 576, 64), (40, 72, 24), (9, 2048, 1024),
+                                   (8200, 520, 8), (16390, 480, 32), (4106, 1664, 128)])
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
 def test_quantizers_edges(rng, N, K, g, dtype):
+    """Blocks of 4 rows (small matrices) and of 64, ends inside a block or a word
+    group, and the per-group kernels."""
     import mmfp4
     w = _crafted(rng, N, K, dtype)
     announce(f"quantizers N={N} K={K} g={g} {dtype.__name__}")
@@ -252,6 +255,47 @@ def test_quantize_fp4_wide_float32_groups(rng, e):
     packed, s = mmfp4.quantize_fp4(to_dev(w), group_size=g)
     assert np.array_equal(to_np(s).view(np.uint16), rs.view(np.uint16))
     assert np.array_equal(to_np(packed).view(np.uint32), rp)
+
+
+def _queued_us(call, n=40):
+    """Median GPU time of a call with the launches queued ahead."""
+    call()
+    times = []
+    for _ in range(7):
+        torch.cuda._sleep(1_000_000)
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(n):
+            call()
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b) * 1000 / n)
+    return sorted(times)[3]
+
+
+@pytest.mark.parametrize("N,K,g", [(33, 1024, 8), (4, 512, 8), (256, 256, 32)])
+def test_small_quantizers_tiled_form_is_not_slower(N, K, g):
+    """Small matrices through the tiled quantizers and (weights that are not 16-byte
+    aligned) the per-group ones: INT4 33 x 1024 in groups of 8 2.4 against 2.6 us; 9.0
+    in blocks of 64 rows."""
+    import mmfp4
+    lib = mmfp4._lib
+    w = (torch.randn(N * K + 8, device="cuda") * 0.02).half()
+    p = torch.empty(K // 8, N, device="cuda", dtype=torch.int32)
+    s, z = (torch.empty(K // g, N, device="cuda", dtype=torch.float16) for _ in range(2))
+    st = lib.stream_of(s)
+
+    def u4(first):
+        lib.call("mm_u4_quantize", lib.ptr(w[first:]), N, K, g, lib.ptr(p), lib.ptr(s),
+                 lib.ptr(z), st)
+
+    def fp4(first):
+        lib.call("mm_fp4_quantize", lib.ptr(w[first:]), 0, N, K, g, lib.ptr(p), lib.ptr(s), st)
+
+    announce(f"small quantizers N={N} K={K} g={g}")
+    for quantize in (u4, fp4):
+        tiled, per_group = (_queued_us(lambda f=f: quantize(f)) for f in (0, 1))
+        assert tiled < 1.2 * per_group, f"{quantize.__name__}: {tiled:.2f}, {per_group:.2f} us"
 
 
 def test_dequant_wide_form_is_not_slower():
