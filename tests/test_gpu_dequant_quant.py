@@ -220,17 +220,18 @@ def test_quantizers_edges(rng, N, K, g, dtype):
         assert np.array_equal(to_np(z), rz)
 
 
-@pytest.mark.parametrize("N", [1, 4, 64, 255, 576, 1020, 1028])
-def test_dequant_widths(rng, N):
-    """Four columns per thread (N % 4 == 0), with whole lines (N % 64 == 0) and
-    without, and one."""
+@pytest.mark.parametrize("K,N", [(64, 1), (64, 4), (64, 64), (64, 255), (64, 1020), (544, 4096),
+                                 (512, 4096), (1024, 2052), (4096, 516), (8224, 260)])
+def test_dequant_widths(rng, K, N):
+    """Four columns per thread (N % 4 == 0, from 65536 such threads), with whole lines
+    (N % 64 == 0) and without, and one."""
     import mmfp4
-    K, g = 64, 32
+    g = 32
     packed = rng.integers(0, 2**32, (K // 8, N), dtype=np.uint64).astype(np.uint32)
     s = rng.normal(0, 0.01, (K // g, N)).astype(np.float16)
-    s[0, 0], s[1, N - 1] = np.inf, np.nan
+    s[0, 0], s[-1, N - 1] = np.inf, np.nan
     z = rng.integers(0, 16, (K // g, N)).astype(np.float16)
-    announce(f"dequant N={N}")
+    announce(f"dequant K={K} N={N}")
     out = to_np(mmfp4.dequant_fp4(to_dev(packed), to_dev(s), K, N, g))
     assert np.array_equal(out.view(np.uint16), ofp4.dequant_fp4(packed, s, g).view(np.uint16))
     out = to_np(mmfp4.dequant_int4(to_dev(packed), to_dev(s), to_dev(z), K, N, g))
@@ -298,12 +299,15 @@ def test_small_quantizers_tiled_form_is_not_slower(N, K, g):
         assert tiled < 1.2 * per_group, f"{quantize.__name__}: {tiled:.2f}, {per_group:.2f} us"
 
 
-def test_dequant_wide_form_is_not_slower():
-    """Four words per thread against one (scales that are not 8-byte aligned) into a
-    destination that is used again, at a width whose rows end inside a cache line:
-    13.0 against 14.1 us; 16.4 with stores that bypassed the caches."""
+@pytest.mark.parametrize("K,N", [(5376, 4516), (1024, 100)])
+def test_dequant_wide_form_is_not_slower(K, N):
+    """Operands that allow four words per thread against one word per thread (scales
+    that are not 8-byte aligned) into a destination that is used again.  At a width
+    whose rows end inside a cache line 13.0 against 14.1 us, 16.4 with stores that
+    bypassed the caches; a small matrix takes one word per thread either way, 2.0 us
+    (2.4 with four)."""
     import mmfp4
-    K, N, g = 5376, 4516, 32
+    g = 32
     p = torch.randint(-2**31, 2**31 - 1, (K // 8, N), device="cuda", dtype=torch.int32)
     s = torch.full((K // g * N + 4,), 0.01, device="cuda", dtype=torch.float16)
     z = torch.full((K // g, N), 7.0, device="cuda", dtype=torch.float16)
@@ -311,19 +315,10 @@ def test_dequant_wide_form_is_not_slower():
     lib = mmfp4._lib
 
     def us(first):
-        sv = s[first:first + K // g * N]
-        times = []
-        for _ in range(8):
-            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-            a.record()
-            for _ in range(50):
-                lib.call("mm_u4_dequant", lib.ptr(p), lib.ptr(sv), lib.ptr(z), lib.ptr(out), K, N,
-                         g, lib.stream_of(out))
-            b.record()
-            b.synchronize()
-            times.append(a.elapsed_time(b) * 20)
-        return min(times)
+        sv, st = s[first:first + K // g * N], lib.stream_of(out)
+        return _queued_us(lambda: lib.call("mm_u4_dequant", lib.ptr(p), lib.ptr(sv), lib.ptr(z),
+                                           lib.ptr(out), K, N, g, st))
 
     announce(f"dequant forms K={K} N={N}")
     one, four = us(1), us(0)
-    assert four < 1.05 * one, f"{four:.2f} us with four words per thread, {one:.2f} with one"
+    assert four < 1.12 * one, f"{four:.2f} us with four words per thread, {one:.2f} with one"
