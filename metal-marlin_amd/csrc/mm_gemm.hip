@@ -1439,10 +1439,14 @@ int multi_dispatch(const char* who, const f16* A, int nmat, const uint32_t* cons
   MM_CHECK_ARG((al & 15) == 0, "%s: A, B 16-byte / scales, C 8-byte alignment required", who);
   MM_CHECK_ARG(tiles <= SK_MAX_TILES, "%s: too many columns", who);
   if (M == 0) return 0;
-  // Two-slab kernel where one product of the same width takes it (4096 ->
-  // 4096 + 1024 + 1024 at M = 1, against 64-column tiles: a layer's four calls
-  // 32.3 -> 31.3 us).
-  if (use_dual(M, ntot, K, g))
+  // Two-slab kernel where one product of the same width takes it, and its waves are
+  // filled: each takes 512 k of a round, so up to K = 2048 a part-filled wave is a
+  // large share.  us on 64-column tiles -> two-slab, 3072 columns, M = 1 and 8:
+  // K = 512 3.3 -> 3.5, 3.3 -> 3.6 (g = 64); 1024 3.6, 3.6 -> 3.75; 1536 3.9 -> 3.6,
+  // 4.1 -> 3.9 (g = 128); 1792 4.0, 4.3 -> 4.6; 2048 4.0 -> 3.6, 4.5 -> 4.2; 2304 5.6
+  // -> 4.25, 6.2 -> 5.0; 4096 -> 4096 + 1024 + 1024 at M = 1 a layer's four calls
+  // 32.3 -> 31.3.
+  if (use_dual(M, ntot, K, g) && (K > 2048 || (K % 512 == 0 && K >= 1536)))
     return launch_dual_multi(A, M, K, g, st, &mp);
   if (M > 16)
     return launch_skinny<false, 2, SK_MULTI>(A, K, nullptr, nullptr, nullptr, nullptr, nullptr,

@@ -423,9 +423,12 @@ def test_multi_qkv_two_row_blocks(rng, M):
 
 
 @pytest.mark.parametrize("M,K,Ns", [(1, 4096, (4096, 1024, 1024)), (8, 2048, (3004, 36, 64)),
-                                    (5, 4160, (2048, 1028, 4))])
+                                    (5, 4160, (2048, 1028, 4)), (8, 1536, (2052, 1024, 8)),
+                                    (8, 1792, (2052, 1024, 8)), (2, 512, (1024, 1024, 1028)),
+                                    (3, 2112, (1024, 1024, 1028))])
 def test_multi_qkv_two_slab(rng, M, K, Ns):
-    """The two-slab kernel over three matrices, widths that end inside a tile."""
+    """The two-slab kernel over three matrices, widths that end inside a tile, and
+    the sizes of K around those that it takes."""
     import mmfp4
     g = 64
     w = [_exact_fp4(rng, K, n, g) for n in Ns]
