@@ -71,9 +71,9 @@ struct SkMulti {
 // fp32 with PW = N, 2N for the pair modes (gate at n, up at N + n), or ntot.
 // ROWP: 0 Marlin-layout weights; 1, 2 row-packed [N, K/8] weights with
 // scales [N, K/g] (1) or [K/g, N] (2), transposed through LDS into the
-// Marlin operand order (skinny_wave RT) or, the pair at up to 16 rows with groups
-// of 128 or a multiple of 256 k, read in place from LDS (skinny_wave_rows);
-// 3 Marlin-layout weights with scales [N, K/g].
+// Marlin operand order (skinny_wave RT); 3 Marlin-layout weights with scales
+// [N, K/g]; 4 as 2 (the pair at up to 16 rows, groups of 128 or a multiple of 256 k,
+// pair_rows_form), the words read in place from LDS (skinny_wave_rows).
 // Row-packed single-tile blocks: the RT staging takes a few registers over
 // the 128 that keep two 8-wave blocks resident per CU; at that limit the
 // flush intervals listed here compile without spills (the others keep the
@@ -97,7 +97,7 @@ k_skinny(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
   constexpr bool ONE = ACT == SK_PLAIN || ACT == SK_MULTI;   // one matrix per block
   // Row-packed weights are staged through 8 KiB of LDS per wave and tile in
   // the main loop; the block reduction reuses the same memory afterwards.
-  constexpr bool STAGE = ROWP == 1 || ROWP == 2;
+  constexpr bool STAGE = ROWP == 1 || ROWP == 2 || ROWP == 4;
   // 9..32 rows, one column tile: each wave's activation slab (16*MT rows x
   // 32*SPW k, 8 KiB) goes through LDS too, when every round lies inside K
   // (measured on MI355X, per Llama layer: M=16 46.6 -> 44.6 us, M=32
@@ -149,7 +149,7 @@ k_skinny(const f16* __restrict__ A, int lda, const uint32_t* __restrict__ B,
                 : (t == 0 ? SkTile{B, S, Z, n0} : SkTile{B2, S2, Z2, n0});
   if constexpr (STAGE) {
     static_assert(!INT4 && ACT != SK_MULTI, "row-packed: FP4 product or gate/up pair");
-    if constexpr (!ONE && ROWP == 2 && MT == 1 && SPW == 8 && FL >= 4)
+    if constexpr (ROWP == 4)
       skinny_wave_rows<FL>(A, lda, M, tl, N, K, g, blk_st0 + wave * SPW, nrounds, NW * SPW, acc,
                            (char*)red + wave * NT * 8192);
     else skinny_wave<false, MT, NT, SPW, FL, false, ROWP == 1, false, true>(
@@ -913,6 +913,23 @@ size_t skinny_ws_bytes(int M, int N, int K) {
 // B2/S2/Z2 the up matrix, both [.., N]; the split and workspace are those of
 // the unfused [K, 2N] product (plan_skinny(M, 2N, K)).
 // SK_MULTI: `mp` describes the matrices (N is then mp->ntot, B..Z2 unused).
+// Whether the row-packed pair reads its words in place from LDS (skinny_wave_rows)
+// rather than transposing them (RT).  In place, an activation load touches four lines
+// per row where RT's order touches one, and the loads of a wave's next round travel
+// during the math: better with few rows and with several rounds, and in a single one
+// where not all waves have work.  us, RT -> in place, g = 128:
+//   one round    1024 -> 2 x 2816 M = 1 5.0 -> 4.6, M = 16 5.2 -> 5.4; with all waves
+//                at work, 2048 -> 2 x 8192 2% slower from M = 1 on
+//   two rounds   4096 -> 2 x 11008 M = 1 13.6 -> 12.4, M = 10 6% and M = 12 3% faster, M
+//                = 16 15.1 -> 15.2; 3072 -> 2 x 8192 M = 10 0.6% and M = 12 2% slower
+//   three        6144 -> 2 x 16384 M = 10 1% and M = 16 4% slower, 5120 -> 2 x 13824 4%
+//                faster both (g = 512)
+//   four         8192 -> 2 x 28672 M = 1 52.4 -> 47.8, M = 16 57.2 -> 55.8
+bool pair_rows_form(int M, int K, const SkinnyPlan& p, int slab) {
+  if (p.nrounds == 1) return M <= 4 && K < 32 * slab * p.ksplit;
+  return M <= 10 || p.nrounds >= 4;
+}
+
 #define MM_ROWP_TILES 1      // 64-column tiles per block of the plain row-packed product; 2
                              // measured slower at M=1 (4096x6144 10.1 -> 18.8 us)
 template <int INT4, int MT, int ACT, int ROWP = 0>
@@ -952,6 +969,15 @@ int launch_skinny(const f16* A, int lda, const uint32_t* B, const f16* S, const 
     case 4: MM_LAUNCH_SK(4 <= SPW ? 4 : 0, RP); break;                                      \
     case 8: MM_LAUNCH_SK(8 <= SPW ? 8 : 0, RP); break;                                      \
     default: MM_LAUNCH_SK(0, RP); break;                                                    \
+  }
+  if constexpr ((ACT == SK_SWIGLU || ACT == SK_PAIR) && MT == 1 && ROWP == 2) {
+    static_assert(SPW == 8, "a round is 8 pieces of a column");
+    if ((fl == 4 || fl == 8) && pair_rows_form(M, K, p, sk_nw<MT>() * SPW)) {
+      if (fl == 4) MM_LAUNCH_SK(4, 4);
+      else MM_LAUNCH_SK(8, 4);
+      MM_CHECK_LAUNCH("gemm(skinny)");
+      return 0;
+    }
   }
   MM_LAUNCH_SK_FL(ROWP)
 #undef MM_LAUNCH_SK_FL

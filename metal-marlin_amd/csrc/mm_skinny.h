@@ -417,7 +417,8 @@ MM_DEV void skinny_wave(const f16* __restrict__ A, int lda, const int* __restric
 // Piece p of column 4c + j lies at 16-byte unit 8 * (16 * j + c) + (p ^ (c >> 1)):
 // the 16 lanes of an LDS read pass hit all banks.
 // Measured against RT, 4096 -> 2 x 14336, g = 128: M = 1 15.7 -> 14.1 us, M = 8
-// 16.0 -> 15.0, M = 16 16.4 both.  RT stays for the rest: with g = 64 the two are
+// 16.0 -> 15.0, M = 16 16.4 both.  RT stays where rows are many and rounds few
+// (pair_rows_form), and for the rest: with g = 64 the two are
 // equal (and this form spills registers at g = 32); single-tile products and
 // the pair at 17..32 rows are slower in this form (14336 -> 4096 M = 16 12.3 ->
 // 13.2, pair M = 32 22.7 -> 25.4: an activation load touches four lines per row

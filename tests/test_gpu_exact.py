@@ -442,11 +442,14 @@ def test_multi_qkv_two_slab(rng, M, K, Ns):
 @pytest.mark.parametrize("M,K,N,g", [
     (1, 128, 8, 128), (2, 384, 72, 128), (7, 4096, 1032, 128), (16, 2176, 200, 128),
     (15, 2560, 136, 256), (9, 1024, 6408, 512), (3, 14336, 64, 1024),
+    (4, 1920, 520, 128), (5, 2048, 520, 128), (10, 4096, 3080, 128), (7, 2304, 3080, 256),
+    (11, 4096, 3080, 128), (16, 6272, 3080, 128),
 ])
 def test_rowpacked_pair_decode(rng, M, K, N, g):
-    """Row-packed pair at decode sizes, groups of 128 and more: rounds that
-    overhang K, columns that end inside a tile, one and several rounds per wave,
-    with and without a K split."""
+    """Row-packed pair at decode sizes, groups of 128 and more, words read in place
+    from LDS or transposed (by rows and rounds per wave): rounds that overhang K,
+    columns that end inside a tile, one and several rounds per wave, with and
+    without a K split."""
     import mmfp4
     w = [_exact_fp4(rng, K, N, g) for _ in range(2)]
     a = _acts(rng, M, K)
