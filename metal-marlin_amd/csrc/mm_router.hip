@@ -99,25 +99,15 @@ MM_DEV void wave_argmax(float& v, int& i) {
   i = key_index(k);
 }
 
-// Where the selected probabilities go: fp32, or fp16 (rounded once from the
-// fp32 value, which is what a caller's conversion launch would store; that
-// launch cost 4 us, as much as the top-k itself at a few tokens).
-struct ProbOut {
-  float* f32;
-  f16* h;
-  MM_DEV void put(size_t i, float v) const {
-    if (f32 != nullptr) f32[i] = v;
-    else h[i] = (f16)v;
-  }
-  MM_DEV ProbOut at(size_t o) const {
-    return ProbOut{f32 ? f32 + o : nullptr, h ? h + o : nullptr};
-  }
-};
+// PT: the probabilities are stored as fp32, or as fp16 (rounded once from the fp32
+// value, which is what a caller's conversion launch would store; that launch cost
+// 4 us, as much as the top-k itself at a few tokens).
 
 // One wave: softmax + top-k of one token's logits row `lg` (fp32, E
 // entries, already rounded as the reference rounds them) -> ids / probs.
+template <typename PT>
 MM_DEV void softmax_topk_row(const float* lg, int E, int k, int renorm, int64_t* ids,
-                             ProbOut probs) {
+                             PT* probs) {
   const int lane = threadIdx.x & 63;
   float mx = -INFINITY;
   for (int e = lane; e < E; e += 64) mx = fmaxf(mx, lg[e]);
@@ -154,7 +144,7 @@ MM_DEV void softmax_topk_row(const float* lg, int E, int k, int renorm, int64_t*
   }
   if (lane < k) {
     ids[lane] = my_i;
-    probs.put(lane, renorm ? my_p / taken_sum : my_p);
+    probs[lane] = (PT)(renorm ? my_p / taken_sum : my_p);
   }
 }
 
@@ -164,9 +154,9 @@ MM_DEV void softmax_topk_row(const float* lg, int E, int k, int renorm, int64_t*
 // expression and summation order as softmax_topk_row) and kept in registers;
 // a round is then one register scan and one wave arg-max per row.  Rows
 // j >= nvalid are computed but not stored.
-template <int NR, int SL>
+template <int NR, int SL, typename PT>
 MM_DEV void softmax_topk_rows(const float* lg, int rstride, int nvalid, int E, int k, int renorm,
-                              int64_t* ids, ProbOut probs) {
+                              int64_t* ids, PT* probs) {
   const int lane = threadIdx.x & 63;
   float p[NR][SL], mx[NR], sm[NR];
 #pragma unroll
@@ -243,7 +233,7 @@ MM_DEV void softmax_topk_rows(const float* lg, int rstride, int nvalid, int E, i
     for (int j = 0; j < NR; ++j) {
       if (j >= nvalid) break;
       ids[j * k + lane] = my_i[j];
-      probs.put(j * k + lane, renorm ? my_p[j] / taken[j] : my_p[j]);
+      probs[j * k + lane] = (PT)(renorm ? my_p[j] / taken[j] : my_p[j]);
     }
   }
 }
@@ -273,9 +263,9 @@ MM_DEV float row_sum(float v) {
 }
 
 // ld(j, e): logit e of row j (e < E).
-template <int SL, class Ld>
+template <int SL, class Ld, typename PT>
 MM_DEV void softmax_topk_rows16(Ld ld, int nvalid, int E, int k, int renorm, int64_t* ids,
-                                ProbOut probs) {
+                                PT* probs) {
   const int lane = threadIdx.x & 63;
   const int j = lane >> 4, l = lane & 15;
   float p[SL];
@@ -335,7 +325,7 @@ MM_DEV void softmax_topk_rows16(Ld ld, int nvalid, int E, int k, int renorm, int
       const int r = 16 * s + l;
       if (r < k) {
         ids[j * k + r] = my_i[s];
-        probs.put(j * k + r, renorm ? my_p[s] / taken : my_p[s]);
+        probs[j * k + r] = (PT)(renorm ? my_p[s] / taken : my_p[s]);
       }
     }
   }
@@ -360,11 +350,11 @@ inline int rt_slots(int E) {
 // Slice partials go to the workspace with agent-scope stores; the last block
 // of a token block to arrive sums them in slice order, adds the bias, rounds
 // the logits to fp16 in LDS and runs softmax + top-k, one wave per token.
-template <bool R16, int SL>
+template <bool R16, int SL, typename PT>
 __global__ void __launch_bounds__(RT_NW * 64)
 k_moe_router(const f16* __restrict__ X, const f16* __restrict__ W, const float* __restrict__ bias,
              int T, int H, int E, int k, int renorm, int spl, int nsl, float* __restrict__ part,
-             uint32_t* __restrict__ counters, int64_t* __restrict__ ids, ProbOut probs) {
+             uint32_t* __restrict__ counters, int64_t* __restrict__ ids, PT* __restrict__ probs) {
   extern __shared__ float lg[];                 // [RT_TOK][E]
   __shared__ uint32_t s_last;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -450,10 +440,10 @@ k_moe_router(const f16* __restrict__ X, const f16* __restrict__ W, const float* 
     if constexpr (R16)
       softmax_topk_rows16<SL>([&](int j, int e) { return lg[(r0 + j) * E + e]; },
                               min(NR, T - t0 - r0), E, k, renorm, ids + (size_t)(t0 + r0) * k,
-                              probs.at((size_t)(t0 + r0) * k));
+                              probs + (size_t)(t0 + r0) * k);
     else
       softmax_topk_rows<NR, SL>(lg + r0 * E, E, min(NR, T - t0 - r0), E, k, renorm,
-                                ids + (size_t)(t0 + r0) * k, probs.at((size_t)(t0 + r0) * k));
+                                ids + (size_t)(t0 + r0) * k, probs + (size_t)(t0 + r0) * k);
   }
   if (threadIdx.x == 0)
     __hip_atomic_store(&counters[tb], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -476,10 +466,10 @@ RouterPlan plan_router(int H, int E) {
 // Softmax + top-k of given logits [T, E] (fp16 or fp32).  SL > 0 (E <= 1024):
 // RT_WAVES waves x NR tokens per block, NR rows per wave at once; SL == 0:
 // one token per wave, probabilities recomputed per round.
-template <int NR, int SL, bool R16>
+template <int NR, int SL, bool R16, typename PT>
 __global__ void __launch_bounds__(RT_WAVES * 64)
 k_softmax_topk(const void* __restrict__ logits, int logits_f32, int T, int E, int k, int renorm,
-               int64_t* __restrict__ ids, ProbOut probs) {
+               int64_t* __restrict__ ids, PT* __restrict__ probs) {
   extern __shared__ float lg[];                 // [RT_WAVES][NR][E]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t0 = (blockIdx.x * RT_WAVES + wave) * NR;
@@ -493,13 +483,13 @@ k_softmax_topk(const void* __restrict__ logits, int logits_f32, int T, int E, in
     if (logits_f32)
       softmax_topk_rows16<SL>(
           [&](int j, int e) { return ((const float*)logits)[base + (size_t)min(j, jmax) * E + e]; },
-          nv, E, k, renorm, ids + (size_t)t0 * k, probs.at((size_t)t0 * k));
+          nv, E, k, renorm, ids + (size_t)t0 * k, probs + (size_t)t0 * k);
     else
       softmax_topk_rows16<SL>(
           [&](int j, int e) {
             return (float)((const f16*)logits)[base + (size_t)min(j, jmax) * E + e];
           },
-          nv, E, k, renorm, ids + (size_t)t0 * k, probs.at((size_t)t0 * k));
+          nv, E, k, renorm, ids + (size_t)t0 * k, probs + (size_t)t0 * k);
     return;
   }
   float* rows = lg + (size_t)wave * NR * E;
@@ -508,10 +498,10 @@ k_softmax_topk(const void* __restrict__ logits, int logits_f32, int T, int E, in
       rows[j * E + e] = logits_f32 ? ((const float*)logits)[(size_t)(t0 + j) * E + e]
                                    : (float)((const f16*)logits)[(size_t)(t0 + j) * E + e];
   if constexpr (SL == 0) {
-    softmax_topk_row(rows, E, k, renorm, ids + (size_t)t0 * k, probs.at((size_t)t0 * k));
+    softmax_topk_row(rows, E, k, renorm, ids + (size_t)t0 * k, probs + (size_t)t0 * k);
   } else {
     softmax_topk_rows<NR, SL>(rows, E, nv, E, k, renorm, ids + (size_t)t0 * k,
-                              probs.at((size_t)t0 * k));
+                              probs + (size_t)t0 * k);
   }
 }
 
@@ -527,8 +517,9 @@ extern "C" size_t mm_moe_router_workspace_bytes(int T, int H, int E) {
          (size_t)mm_cdiv(T, RT_TOK) * p.nsl * RT_TOK * E * sizeof(float);
 }
 
+template <typename PT>
 static int router(const uint16_t* X, const uint16_t* W, const float* bias, int T, int H, int E,
-                  int k, int renorm, int64_t* ids, ProbOut probs, void* ws, size_t ws_bytes,
+                  int k, int renorm, int64_t* ids, PT* probs, void* ws, size_t ws_bytes,
                   void* stream) {
   MM_CHECK_ARG(T >= 0 && H > 0 && E > 0, "mm_moe_router: bad shape T=%d H=%d E=%d", T, H, E);
   MM_CHECK_ARG(H % 32 == 0, "mm_moe_router: hidden size %d must be divisible by 32", H);
@@ -548,7 +539,7 @@ static int router(const uint16_t* X, const uint16_t* W, const float* bias, int T
   const size_t lds = (size_t)RT_TOK * E * sizeof(float);
   float* part = (float*)((char*)ws + (size_t)RT_MAX_TB * sizeof(uint32_t));
 #define MM_LAUNCH_RT(R16, SLV)                                                                 \
-  hipLaunchKernelGGL((k_moe_router<R16, SLV>), dim3(p.nbx, mm_cdiv(T, RT_TOK)), dim3(RT_NW * 64), \
+  hipLaunchKernelGGL((k_moe_router<R16, SLV, PT>), dim3(p.nbx, mm_cdiv(T, RT_TOK)), dim3(RT_NW * 64), \
                      lds, (hipStream_t)stream, (const f16*)X, (const f16*)W, bias, T, H, E, k,     \
                      renorm, p.spl, p.nsl, part, (uint32_t*)ws, ids, probs)
   switch (rt16_slots(E)) {
@@ -569,18 +560,18 @@ static int router(const uint16_t* X, const uint16_t* W, const float* bias, int T
 extern "C" int mm_moe_router(const uint16_t* X, const uint16_t* W, const float* bias, int T, int H,
                              int E, int k, int renorm, int64_t* ids, float* probs, void* ws,
                              size_t ws_bytes, void* stream) {
-  return router(X, W, bias, T, H, E, k, renorm, ids, ProbOut{probs, nullptr}, ws, ws_bytes, stream);
+  return router(X, W, bias, T, H, E, k, renorm, ids, probs, ws, ws_bytes, stream);
 }
 
 extern "C" int mm_moe_router_p16(const uint16_t* X, const uint16_t* W, const float* bias, int T,
                                  int H, int E, int k, int renorm, int64_t* ids, uint16_t* probs,
                                  void* ws, size_t ws_bytes, void* stream) {
-  return router(X, W, bias, T, H, E, k, renorm, ids, ProbOut{nullptr, (f16*)probs}, ws, ws_bytes,
-                stream);
+  return router(X, W, bias, T, H, E, k, renorm, ids, (f16*)probs, ws, ws_bytes, stream);
 }
 
+template <typename PT>
 static int softmax_topk(const void* logits, int logits_f32, int T, int E, int k, int renorm,
-                        int64_t* ids, ProbOut probs, void* stream) {
+                        int64_t* ids, PT* probs, void* stream) {
   MM_CHECK_ARG(T >= 0 && E > 0, "mm_softmax_topk: bad shape T=%d E=%d", T, E);
   MM_CHECK_ARG(E <= 64 * 64, "mm_softmax_topk: num_experts=%d must be <= 4096", E);
   MM_CHECK_ARG(k >= 1 && k <= RT_MAXK && k <= E, "mm_softmax_topk: top_k=%d must be in [1, %d]",
@@ -592,7 +583,7 @@ static int softmax_topk(const void* logits, int logits_f32, int T, int E, int k,
   const size_t lds = sl16 > 0 ? 0 : (size_t)RT_WAVES * nr * E * sizeof(float);
   const dim3 grid(mm_cdiv(T, RT_WAVES * nr));
 #define MM_LAUNCH_ST(NRV, SLV, R16)                                                              \
-  hipLaunchKernelGGL((k_softmax_topk<NRV, SLV, R16>), grid, dim3(RT_WAVES * 64), lds,             \
+  hipLaunchKernelGGL((k_softmax_topk<NRV, SLV, R16, PT>), grid, dim3(RT_WAVES * 64), lds,             \
                      (hipStream_t)stream, logits, logits_f32, T, E, k, renorm, ids, probs)
   switch (sl16) {
     case 1: MM_LAUNCH_ST(4, 1, true); break;
@@ -612,11 +603,10 @@ static int softmax_topk(const void* logits, int logits_f32, int T, int E, int k,
 
 extern "C" int mm_softmax_topk(const void* logits, int logits_f32, int T, int E, int k,
                                int renorm, int64_t* ids, float* probs, void* stream) {
-  return softmax_topk(logits, logits_f32, T, E, k, renorm, ids, ProbOut{probs, nullptr}, stream);
+  return softmax_topk(logits, logits_f32, T, E, k, renorm, ids, probs, stream);
 }
 
 extern "C" int mm_softmax_topk_p16(const void* logits, int logits_f32, int T, int E, int k,
                                    int renorm, int64_t* ids, uint16_t* probs, void* stream) {
-  return softmax_topk(logits, logits_f32, T, E, k, renorm, ids, ProbOut{nullptr, (f16*)probs},
-                      stream);
+  return softmax_topk(logits, logits_f32, T, E, k, renorm, ids, (f16*)probs, stream);
 }
