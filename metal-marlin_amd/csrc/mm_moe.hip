@@ -654,12 +654,14 @@ k_moe_prefill(const f16* __restrict__ X, const int32_t* __restrict__ sorted_idx,
 // columns per thread.  nvalid (may be null): the sort's count of valid
 // assignments; slots placed at or past it (dropped ids) contribute nothing.
 // PT: fp32 or fp16 probabilities (fp16 ones are exact in fp32, so callers that
-// hold them need no conversion launch: 4 us each way).  The slots' rows are
-// loaded CMB_U at a time, and a wave loads its token's weights once, one per
-// lane.  T = 32, H = 2048, k = 8: 4.9 us one row at a time, 4.0 so (T = 1024 7.8,
-// 8.0).
-constexpr int CMB_U = 4;
-template <typename PT>
+// hold them need no conversion launch: 4 us each way).  The slots' rows are loaded U
+// at a time, U = 1 or 2 where there are no more, 3 where it divides k, else 4: T = 32,
+// H = 2048, k = 8 3.4 us one row at a time, 3.0 so (T = 1024 6.2, 5.5).  Above 2048
+// tokens (eight blocks per CU) the blocks hide each other's latency and U = 1 is up to
+// 7% faster (T = 3000, H = 1024, k = 3 4.3 us, 4.6).  From three slots on a wave loads
+// its token's weights once, one per lane; with one or two that only delays the rows,
+// and so does loading four rows for them (T = 3000, H = 1024, k = 1 3.3 us, 4.3).
+template <typename PT, int U>
 __global__ void __launch_bounds__(256)
 k_moe_combine(const f16* __restrict__ Y, const PT* __restrict__ probs,
               const int32_t* __restrict__ inverse, int k, int kin, float wsh,
@@ -670,8 +672,9 @@ k_moe_combine(const f16* __restrict__ Y, const PT* __restrict__ probs,
   // Lane l of every wave holds the weight of slot l (all lanes load: the column
   // loop below may leave some idle); slots past 63 are loaded when used.
   auto load_weight = [&](int j) { return j < kin ? (float)probs[(size_t)t * kin + j] : wsh; };
-  const int lane_w = __builtin_bit_cast(int, load_weight(threadIdx.x & 63));
+  const int lane_w = U < 3 ? 0 : __builtin_bit_cast(int, load_weight(threadIdx.x & 63));
   auto weight = [&](int j) {
+    if (U < 3) return load_weight(j);
     return j < 64 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(lane_w, j))
                   : load_weight(j);
   };
@@ -682,17 +685,17 @@ k_moe_combine(const f16* __restrict__ Y, const PT* __restrict__ probs,
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = (float)b[i];
     }
-    for (int j0 = 0; j0 < k; j0 += CMB_U) {
-      int r[CMB_U];
-      f16x8 y[CMB_U];
+    for (int j0 = 0; j0 < k; j0 += U) {
+      int r[U];
+      f16x8 y[U];
 #pragma unroll
-      for (int u = 0; u < CMB_U; ++u) r[u] = inverse[(size_t)t * k + min(j0 + u, k - 1)];
+      for (int u = 0; u < U; ++u) r[u] = inverse[(size_t)t * k + min(j0 + u, k - 1)];
       // Unconditional loads (row 0 in place of a dropped one), so all are in flight.
 #pragma unroll
-      for (int u = 0; u < CMB_U; ++u)
+      for (int u = 0; u < U; ++u)
         y[u] = *(const f16x8*)(Y + (size_t)(r[u] < lim ? r[u] : 0) * H + 8 * h8);
 #pragma unroll
-      for (int u = 0; u < CMB_U; ++u)
+      for (int u = 0; u < U; ++u)
         if (j0 + u < k && r[u] < lim) {
           const float p = weight(j0 + u);
 #pragma unroll
@@ -848,8 +851,15 @@ int combine(const uint16_t* Y, const PT* probs, const int32_t* inverse, int T, i
   MM_CHECK_ARG(T >= 0 && k > 0 && H > 0, "mm_moe_combine: bad shape");
   MM_CHECK_ARG(H % 8 == 0, "mm_moe_combine: H=%d must be divisible by 8", H);
   if (T == 0) return 0;
-  hipLaunchKernelGGL(k_moe_combine<PT>, dim3(T), dim3(256), 0, (hipStream_t)stream, (const f16*)Y,
-                     probs, inverse, k, kin, wsh, (const f16*)base, nvalid, H, (f16*)out);
+#define MM_LAUNCH_COMBINE(U)                                                                      \
+  hipLaunchKernelGGL((k_moe_combine<PT, U>), dim3(T), dim3(256), 0, (hipStream_t)stream,           \
+                     (const f16*)Y, probs, inverse, k, kin, wsh, (const f16*)base, nvalid, H,      \
+                     (f16*)out)
+  if (k == 1 || T > 2048) MM_LAUNCH_COMBINE(1);
+  else if (k == 2) MM_LAUNCH_COMBINE(2);
+  else if (k % 3 == 0) MM_LAUNCH_COMBINE(3);
+  else MM_LAUNCH_COMBINE(4);
+#undef MM_LAUNCH_COMBINE
   MM_CHECK_LAUNCH("mm_moe_combine");
   return 0;
 }

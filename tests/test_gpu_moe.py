@@ -332,10 +332,11 @@ def test_moe_mlp_out_aliases_hidden(rng, T):
     assert torch.equal(xin, want)
 
 
-@pytest.mark.parametrize("T,k,H", [(1, 1, 8), (3, 8, 40), (2, 64, 2008), (2, 70, 512), (5, 6, 4104)])
+@pytest.mark.parametrize("T,k,H", [(1, 1, 8), (3, 8, 40), (2, 64, 2008), (2, 70, 512), (5, 6, 4104),
+                                   (4, 2, 520), (3, 3, 264), (2, 5, 1032), (1, 72, 24), (2049, 5, 24)])
 def test_combine_widths(rng, T, k, H):
     """Combine where the column loop leaves lanes idle (H / 8 not a multiple of
-    64), at and past 64 slots."""
+    64), at and past 64 slots, by one to four slots at a time."""
     import mmfp4
     from mmfp4.moe_dispatch import MoEDispatchInfo
     y = torch.from_numpy(rng.normal(0, 1, (T * k, H)).astype(np.float16)).cuda()
